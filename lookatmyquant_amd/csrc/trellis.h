@@ -9,9 +9,8 @@
 // B (R floats) travel through LDS: member h*R + r has the path cost B((h*R + r) >> K) + (x - C)^2, which
 // its group's owner forms itself with the reference's three rounded operations (difference, square, sum),
 // hence the same float32 value. Per step a thread reads the B entries of its members, forms the NB costs
-// of each of its groups, keeps the minimum and its h (strict comparison in increasing h: the lowest h wins
-// a tie, as torch's min does) and writes its G new minima: R floats written and R read per step, a
-// quarter of the full cost vector.
+// of each of its groups, keeps the minimum and its h (the lowest h wins a tie, as torch's min does: pair_min) and
+// writes its G new minima: R floats written and R read per step, a quarter of the full cost vector.
 #pragma once
 #include "common.h"
 
@@ -140,6 +139,45 @@ struct TabF16 {
         q1 = d1 * d1;
     }
 };
+
+// A group's minimum and the lowest h attaining it, one instruction per member: the float64 whose high word is the cost's
+// bits and whose low word is h orders as (cost, h) does (costs are +0 or above, finite or +inf, so the double is positive
+// and finite), and v_min_f64 keeps the first of the two orders' minima. Why: the searches are bound by vector issue, and
+// on this chip (loops of one instruction, two or more waves a SIMD) an f32 add, subtract, multiply, fma or move and the
+// 32-bit integer add, and, or, xor take 2 clocks a wave, while min, min3, compare, select, add with carry and
+// v_fma_mix take 4, and so does v_min_f64. Four members: three minima and a shift-or, 16 clocks, where the minimum, an
+// equality scan (L <= 12) or a tournament of lane masks (16 bits, k = 2) took 36 and 28, eight 32 against 76, sixteen
+// 64 against 156. Measured: 6,144 x 2,560 at L = 12 and 1 to 4 bits 14.19 -> 13.18 ms, 960 x 960 at L = 16 11.89 ->
+// 10.49 ms, 256 paths of 256 positions at L = 12 114.7 -> 105.7 us. (Forming the costs' sums and differences on the
+// matrix cores, v_mfma_f32_4x4x1, gives the same bits but no time: its clocks add to the vector unit's.) The constants h
+// are opaque to the compiler, which would form them again for every group, and live across the search; each cost is
+// written beside its constant, so the pairs need no moves.
+template <int NB>
+struct LowWords {
+    uint32_t h[NB];
+    __device__ __forceinline__ LowWords()
+    {
+#pragma unroll
+        for (int i = 0; i < NB; ++i) asm volatile("v_mov_b32 %0, %1" : "=v"(h[i]) : "n"(i));
+    }
+};
+__device__ __forceinline__ double cost_and(float c, uint32_t lo) { return __hiloint2double(__float_as_int(c), (int)lo); }
+__device__ __forceinline__ float cost_of(double p) { return __int_as_float(__double2hiint(p)); }
+__device__ __forceinline__ uint32_t low_of(double p) { return (uint32_t)__double2loint(p); }
+
+template <int N>
+__device__ __forceinline__ double pair_min(const float (&c)[N], const LowWords<N>& lo)
+{
+    double m[N / 2];
+#pragma unroll
+    for (int i = 0; i < N / 2; ++i) m[i] = fmin(cost_and(c[2 * i], lo.h[2 * i]), cost_and(c[2 * i + 1], lo.h[2 * i + 1]));
+#pragma unroll
+    for (int w = N / 4; w >= 1; w >>= 1)
+#pragma unroll
+        for (int i = 0; i < N / 4; ++i)
+            if (i < w) m[i] = fmin(m[2 * i], m[2 * i + 1]);
+    return m[0];
+}
 
 // f(IntC<v>{}) for the uniform v in [I, N): a chain of scalar branches, so that f indexes registers statically
 template <int I>
@@ -281,6 +319,7 @@ __device__ int viterbi_gx(const float* xs, int TV, Tab& tab, int start, float* b
 #pragma unroll
             for (int e = 0; e < M; ++e) bv[h][e] = (rs < 0 || d == h * (R >> K) + e) ? 0.0f : __builtin_inff();
     };
+    const LowWords<NB> lo;
     int cur = 0;
     float x = xs[0];
     // From a given start state, position t reaches only the 2^(K (t+1)) states of one aligned range,
@@ -361,56 +400,25 @@ __device__ int viterbi_gx(const float* xs, int TV, Tab& tab, int start, float* b
             tab.hold();
             uint32_t bits = 0;
             float* dst = buf + (DBL ? (cur ^ 1) * R : 0);
-            // groups in chunks of CK sharing one B entry per h (RUN) or all of them; each chunk stored when done
+            // groups in chunks of CK sharing one B entry per h (RUN) or all of them, from the last to the first (the
+            // winning h are shifted in, group 0's last); each chunk stored when done
             constexpr int CK = V::RUN ? NB : G;
-            // with the tournament below (K = 2 in the 16-bit-state kernels) the groups are visited from the last to the
-            // first, so that the winning h can be shifted in bit by bit
-            constexpr bool TOUR = NB == 2 || (NB == 4 && L > 12);
 #pragma unroll
-            for (int ei = 0; ei < G / CK; ++ei) {
-                const int e = TOUR ? G / CK - 1 - ei : ei;
+            for (int e = G / CK - 1; e >= 0; --e) {
                 float best[CK];
 #pragma unroll
-                for (int gi = 0; gi < CK; ++gi) {
-                    const int gg = TOUR ? CK - 1 - gi : gi;
+                for (int gg = CK - 1; gg >= 0; --gg) {
                     const int g = e * CK + gg;
                     float c[NB];
 #pragma unroll
                     for (int h = 0; h < NB; ++h) c[h] = bv[h][e] + tab.dsq(x, h * G + g);
-                    // the minimum, then the lowest h attaining it (costs are never NaN: finite or +inf)
-                    if constexpr (NB == 2) {
-                        // the second state wins only if strictly lower; its bit enters as a carry-in
-                        const uint64_t lo = __builtin_amdgcn_ballot_w64(c[1] < c[0]);
-                        best[gg] = fminf(c[0], c[1]);
-                        bits = shift_in(bits, lo);
-                    } else if constexpr (TOUR) {
-                        // (at L <= 12 the extra register it takes would cost the kernel a wave of occupancy)
-                        // a two-level tournament with strict comparisons (a tie keeps the left, lower, side): the
-                        // winning pair hi = (min(c2,c3) < min(c0,c1)), then within it lo; h = 2 hi + lo enters bits
-                        // [2g, 2g+2) as two carry-ins (bits = 2 bits + bit), the comparisons staying lane masks
-                        // (the minimum as one v_min3 of m01, c2, c3; the right pair wins exactly when it is below m01)
-                        const float m01 = fminf(c[0], c[1]);
-                        const float mb = fminf(m01, fminf(c[2], c[3]));
-                        const uint64_t hi = __builtin_amdgcn_ballot_w64(mb < m01);
-                        const uint64_t lo = (hi & __builtin_amdgcn_ballot_w64(c[3] < c[2])) |
-                                            (~hi & __builtin_amdgcn_ballot_w64(c[1] < c[0]));
-                        best[gg] = mb;
-                        bits = shift_in(bits, hi);
-                        bits = shift_in(bits, lo);
-                    } else {
-                        float b = c[0];
-#pragma unroll
-                        for (int h = 1; h < NB; ++h) b = fminf(b, c[h]);
-                        uint32_t hs = NB - 1;
-#pragma unroll
-                        for (int h = NB - 2; h >= 0; --h) hs = c[h] == b ? (uint32_t)h : hs;
-                        best[gg] = b;
-                        asm volatile("" : "+v"(hs));  // keeps h a small integer: one shift-or per group, no wide constants
-                        bits |= hs << (g * K);
-                    }
+                    const double m = pair_min<NB>(c, lo);
+                    best[gg] = cost_of(m);
+                    bits = (bits << K) | low_of(m);
                 }
                 lds_store_swz<CK>(dst, G * tid + e * CK, best);
             }
+            asm volatile("" : "+v"(bits));  // (32-bit operations above, not the stored width's)
             back[t * V::ACT + tid] = (BackT)bits;
         }
         lds_barrier();

@@ -291,7 +291,7 @@ __device__ __forceinline__ void trellis_block_row(BlkSmem<L, K>& sm, int64_t row
 }
 
 template <int L, int K>
-__global__ __launch_bounds__(LAMQ_NT) void ldlq_trellis_block_kernel(
+__global__ __launch_bounds__(LAMQ_NT, 4) void ldlq_trellis_block_kernel(
     const double* __restrict__ T, int64_t n, int64_t ldT, const double* __restrict__ U, int64_t ldU,
     const double* __restrict__ S, const double* __restrict__ table64, const float* __restrict__ table32,
     int64_t b0, int64_t b1, int width, int look, int32_t* __restrict__ state, int32_t* __restrict__ states,
@@ -361,7 +361,7 @@ constexpr int blk_groups_smem_bytes()
 }
 
 template <int L>
-__global__ __launch_bounds__(LAMQ_NT) void ldlq_trellis_groups_kernel(
+__global__ __launch_bounds__(LAMQ_NT, 4) void ldlq_trellis_groups_kernel(
     const double* __restrict__ T, int64_t n, int64_t ldT, const double* __restrict__ U, int64_t ldU,
     const double* __restrict__ S, int64_t b0, int64_t b1, int width, int look, int32_t* __restrict__ state,
     int32_t* __restrict__ states, int64_t lds, double* __restrict__ Z, int64_t ldZ, int pre, BlkGroups groups)
