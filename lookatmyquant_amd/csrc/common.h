@@ -53,35 +53,35 @@ __device__ __forceinline__ int64_t xcd_remap(int64_t b, int64_t G)
 // fall on 16 different 16-byte bank groups, and reads of consecutive 16-byte chunks stay conflict-free.
 __device__ __forceinline__ int swz(int x) { return x ^ (((x >> 6) & 3) << 2); }
 
-// N floats at logical index x (x a multiple of min(N, 4)), chunk by chunk through swz.
-template <int N>
+// N floats at logical index x (x a multiple of min(N, 4)), chunk by chunk through swz (SWZ false: at x itself).
+template <int N, bool SWZ = true>
 __device__ __forceinline__ void lds_load_swz(const float* __restrict__ base, int x, float (&dst)[N])
 {
     if constexpr (N >= 4) {
 #pragma unroll
         for (int i = 0; i < N; i += 4) {
-            float4 v = *reinterpret_cast<const float4*>(base + swz(x + i));
+            float4 v = *reinterpret_cast<const float4*>(base + (SWZ ? swz(x + i) : x + i));
             dst[i] = v.x; dst[i + 1] = v.y; dst[i + 2] = v.z; dst[i + 3] = v.w;
         }
     } else if constexpr (N == 2) {
-        float2 v = *reinterpret_cast<const float2*>(base + swz(x));
+        float2 v = *reinterpret_cast<const float2*>(base + (SWZ ? swz(x) : x));
         dst[0] = v.x; dst[1] = v.y;
     } else {
-        dst[0] = base[swz(x)];
+        dst[0] = base[SWZ ? swz(x) : x];
     }
 }
 
-template <int N>
+template <int N, bool SWZ = true>
 __device__ __forceinline__ void lds_store_swz(float* __restrict__ base, int x, const float (&src)[N])
 {
     if constexpr (N >= 4) {
 #pragma unroll
         for (int i = 0; i < N; i += 4)
-            *reinterpret_cast<float4*>(base + swz(x + i)) = make_float4(src[i], src[i + 1], src[i + 2], src[i + 3]);
+            *reinterpret_cast<float4*>(base + (SWZ ? swz(x + i) : x + i)) = make_float4(src[i], src[i + 1], src[i + 2], src[i + 3]);
     } else if constexpr (N == 2) {
-        *reinterpret_cast<float2*>(base + swz(x)) = make_float2(src[0], src[1]);
+        *reinterpret_cast<float2*>(base + (SWZ ? swz(x) : x)) = make_float2(src[0], src[1]);
     } else {
-        base[swz(x)] = src[0];
+        base[SWZ ? swz(x) : x] = src[0];
     }
 }
 

@@ -32,6 +32,10 @@ struct VX {
     // h*(R >> K) + M*t. G < NB: one entry per h, (h*R + G*t) >> K, shared by NB/G neighbouring threads.
     static constexpr bool RUN = G >= NB;
     static constexpr int M = RUN ? G / NB : 1;
+    // Up to four groups a thread, its minima are one 16-byte chunk beside its neighbours' and neither the stores nor the
+    // reads meet bank conflicts; a thread of more stores chunks at a stride, spread by swz. Without it every entry a
+    // thread reads lies at one index plus a constant (one address register, not NB).
+    static constexpr bool SWZ = G > 4;
 };
 
 // s_waitcnt lgkmcnt(0) + s_barrier: orders this workgroup's LDS traffic without waiting for its
@@ -165,6 +169,16 @@ __device__ __forceinline__ double cost_and(float c, uint32_t lo) { return __hilo
 __device__ __forceinline__ float cost_of(double p) { return __int_as_float(__double2hiint(p)); }
 __device__ __forceinline__ uint32_t low_of(double p) { return (uint32_t)__double2loint(p); }
 
+// A target as the searches take it: a NaN with its sign cleared, so that the costs it makes are positive NaNs, above every
+// other pair, and an all-NaN group keeps its lowest h (a comparison, which no NaN wins, would too). On the bits, made
+// opaque: the searches are compiled without NaNs, and the compiler would take the test for one and drop it.
+__device__ __forceinline__ float search_target(float x)
+{
+    uint32_t b = (uint32_t)__float_as_int(x);
+    asm volatile("" : "+v"(b));
+    return __int_as_float((int)((b & 0x7FFFFFFFu) > 0x7F800000u ? 0x7FC00000u : b));
+}
+
 template <int N>
 __device__ __forceinline__ double pair_min(const float (&c)[N], const LowWords<N>& lo)
 {
@@ -205,41 +219,27 @@ __device__ __forceinline__ void static_for(F& f)
     }
 }
 
-// Search one path of TV steps; path[0..TV) is complete when this returns (it ends with a barrier).
-//   xs: TV float32 targets (LDS or global). start < 0 leaves the first state free, else only the states
-//   (start << K | b) & (2^L - 1) may begin (codes.py:164-167). buf: DBL ? 2R : R floats of LDS (with one
-//   buffer each step takes a second barrier, between the reads of the old minima and the writes of the new).
-//   back: (TV-1) * ACT entries (LDS or global), entry t*ACT + owner holding the winning h of each of the
-//   owner's groups for the step that produced B_{t+1}. red: 2*(NT/64) words of LDS.
-//   Final state: the lowest among the minimal costs (codes.py:173); traceback codes.py:176-179.
 struct NoHook {
     __device__ __forceinline__ void operator()() const {}
 };
 
-// hook() runs once the forward pass is done (the caller's chance to issue loads that the final argmin and the
-// traceback then cover). BACK_GLOBAL: back-pointers in global memory, published to the tracing thread by a full
-// barrier (otherwise only LDS is ordered, and the caller's outstanding loads stay in flight).
-// lexicographic (v, i) minimum of the wave through DPP moves (no LDS): quad swaps, half-row and row mirrors, then the
-// row broadcasts; lane 63 ends up with the minimum of all 64 lanes.
+// the least pair of the wave through DPP moves (no LDS): quad swaps, half-row and row mirrors, then the row broadcasts;
+// lane 63 ends up with the minimum of all 64 lanes.
 template <int CTRL, int ROWS>
-__device__ __forceinline__ void argmin_dpp(float& v, int& i)
+__device__ __forceinline__ double pair_min_dpp(double p)
 {
-    const float ov = __int_as_float(__builtin_amdgcn_update_dpp(__float_as_int(v), __float_as_int(v), CTRL, ROWS, 0xF, false));
-    const int oi = __builtin_amdgcn_update_dpp(i, i, CTRL, ROWS, 0xF, false);
-    if (ov < v || (ov == v && oi < i)) {
-        v = ov;
-        i = oi;
-    }
+    const int hi = __double2hiint(p), l = __double2loint(p);
+    return fmin(p, __hiloint2double(__builtin_amdgcn_update_dpp(hi, hi, CTRL, ROWS, 0xF, false),
+                                    __builtin_amdgcn_update_dpp(l, l, CTRL, ROWS, 0xF, false)));
 }
-
-__device__ __forceinline__ void wave_argmin(float& v, int& i)
+__device__ __forceinline__ double wave_pair_min(double p)
 {
-    argmin_dpp<0xB1, 0xF>(v, i);   // quad_perm [1,0,3,2]
-    argmin_dpp<0x4E, 0xF>(v, i);   // quad_perm [2,3,0,1]
-    argmin_dpp<0x141, 0xF>(v, i);  // row_half_mirror
-    argmin_dpp<0x140, 0xF>(v, i);  // row_mirror
-    argmin_dpp<0x142, 0xA>(v, i);  // row_bcast15 into rows 1 and 3
-    argmin_dpp<0x143, 0xC>(v, i);  // row_bcast31 into rows 2 and 3
+    p = pair_min_dpp<0xB1, 0xF>(p);   // quad_perm [1,0,3,2]
+    p = pair_min_dpp<0x4E, 0xF>(p);   // quad_perm [2,3,0,1]
+    p = pair_min_dpp<0x141, 0xF>(p);  // row_half_mirror
+    p = pair_min_dpp<0x140, 0xF>(p);  // row_mirror
+    p = pair_min_dpp<0x142, 0xA>(p);  // row_bcast15 into rows 1 and 3
+    return pair_min_dpp<0x143, 0xC>(p);  // row_bcast31 into rows 2 and 3
 }
 
 // the minimum of the wave (float or int) by the same DPP moves; lane 63 ends up with it
@@ -275,20 +275,21 @@ __device__ __forceinline__ int wave_imin(int v)
 // Search one path of TV steps. With PATHREG (TV <= 64) the path comes back in a register of wave 0, lane c holding
 // path[c] (the return value), and is also stored to path[0..TV) (LDS or global); otherwise lane 0 of wave 0 stores
 // path[] as the traceback goes and the return value is 0. Ends with a barrier after which path[] is complete.
-//   xs: TV float32 targets (LDS or global). start < 0 leaves the first state free, else only the states
-//   (start << K | b) & (2^L - 1) may begin (codes.py:164-167). buf: DBL ? 2R : R floats of LDS (with one
-//   buffer each step takes a second barrier, between the reads of the old minima and the writes of the new).
-//   back: (TV-1) * ACT entries (LDS or global), entry t*ACT + owner holding the winning h of each of the
-//   owner's groups for the step that produced B_{t+1}. red: 2*(NT/64) words of LDS.
+//   xs: TV float32 targets (LDS or global), through search_target already or, with RAWX, as they come. start < 0 leaves
+//   the first state free, else only the states (start << K | b) & (2^L - 1) may begin (codes.py:164-167). buf: DBL ? 2R
+//   : R floats of LDS (with one buffer each step takes a second barrier, between the reads of the old minima and the
+//   writes of the new). back: (TV-1) * ACT entries (LDS or global), entry t*ACT + owner holding the winning h of each of
+//   the owner's groups for the step that produced B_{t+1}. red: 2*(NT/64) words of LDS, 8-byte aligned.
 //   Final state: the lowest among the minimal costs (codes.py:173); traceback codes.py:176-179.
 // hook() runs once the forward pass is done (the caller's chance to issue loads that the end of the final argmin and
 // the traceback then cover; at L > 12 after the argmin's two passes over the states). BACK_GLOBAL: back-pointers in
 // global memory, published to the tracing wave by a full barrier (otherwise only LDS is ordered, and the caller's
-// outstanding loads stay in flight).
-template <int L, int K, int NT, bool DBL, bool BACK_GLOBAL = false, bool PATHREG = false, typename BackT, class Tab,
-          class Hook = NoHook>
+// outstanding loads stay in flight). buf_free() runs before the traceback, behind the barrier after which no wave reads
+// or writes buf any more.
+template <int L, int K, int NT, bool DBL, bool BACK_GLOBAL = false, bool PATHREG = false, bool RAWX = false,
+          typename BackT, class Tab, class Hook = NoHook, class BufHook = NoHook>
 __device__ int viterbi_gx(const float* xs, int TV, Tab& tab, int start, float* buf, BackT* back, int* path, float* red,
-                          Hook hook = Hook())
+                          Hook hook = Hook(), BufHook buf_free = BufHook())
 {
     using V = VX<L, K, NT>;
     constexpr int G = V::G, NB = V::NB, M = V::M, R = V::R;
@@ -301,14 +302,16 @@ __device__ int viterbi_gx(const float* xs, int TV, Tab& tab, int start, float* b
 #pragma unroll
     for (int h = 0; h < NB; ++h) ent[h] = V::RUN ? h * (R >> K) + M * tid : (h * R + G * tid) >> K;
     float bv[NB][M];
-    // ent[h] = ent[0] + h (R >> K); where that stride is a multiple of 256 the swizzle keeps it (swz(x + 256 i) =
-    // swz(x) + 256 i), so every h reads at one swizzled index plus a constant offset (one register, not NB)
-    constexpr bool EOFF = (R >> K) % 256 == 0;
+    // ent[h] = ent[0] + h (R >> K), if R >> K entries hold whole neighbourhoods of threads sharing one; where that stride
+    // is a multiple of 256 the swizzle keeps it too (swz(x + 256 i) = swz(x) + 256 i): every h then reads at one index plus
+    // a constant offset (one register, not NB)
+    constexpr bool SWZ = V::SWZ;
+    constexpr bool EOFF = (R >> K) << K == R && (!SWZ || (R >> K) % 256 == 0);
     const auto load_minima = [&](const float* b, int h) {
         if constexpr (EOFF)
-            lds_load_swz<M>(b + h * (R >> K), ent[0], bv[h]);
+            lds_load_swz<M, SWZ>(b + h * (R >> K), ent[0], bv[h]);
         else
-            lds_load_swz<M>(b, ent[h], bv[h]);
+            lds_load_swz<M, SWZ>(b, ent[h], bv[h]);
     };
     // the group minima before position 0: 0 for the start's group (every group with a free start), else +inf
     const auto start_minima = [&]() {
@@ -320,8 +323,9 @@ __device__ int viterbi_gx(const float* xs, int TV, Tab& tab, int start, float* b
             for (int e = 0; e < M; ++e) bv[h][e] = (rs < 0 || d == h * (R >> K) + e) ? 0.0f : __builtin_inff();
     };
     const LowWords<NB> lo;
+    const auto target = [&](int t) { return RAWX ? search_target(xs[t]) : xs[t]; };
     int cur = 0;
-    float x = xs[0];
+    float x = target(0);
     // From a given start state, position t reaches only the 2^(K (t+1)) states of one aligned range,
     // [(start << K (t+1)) mod 2^L, + 2^(K (t+1))); every other state's cost is +inf there, and so is the group minimum
     // in bv of each of them (a state is reachable exactly when a state of its predecessor group is). Two savings follow,
@@ -361,7 +365,7 @@ __device__ int viterbi_gx(const float* xs, int TV, Tab& tab, int start, float* b
     bool live = wave_live(0);
     // one step of the search, position t, reading minima buffer cur (written into cur ^ 1 with two buffers)
     const auto step = [&](const int t, int& cur) {
-        const float xn = xs[t + 1];
+        const float xn = target(t + 1);
         const int base = (SKIP && st0 >= 0 && K * (t + 1) < L)
                              ? (int)(((uint32_t)st0 << (K * (t + 1))) & (uint32_t)(V::NS - 1)) : 0;
         const bool one_h = SKIP && st0 >= 0 && K * (t + 1) <= L - K;
@@ -373,7 +377,7 @@ __device__ int viterbi_gx(const float* xs, int TV, Tab& tab, int start, float* b
 #pragma unroll
             for (int i = 0; i < CKI; ++i) infs[i] = __builtin_inff();
 #pragma unroll
-            for (int e = 0; e < G / CKI; ++e) lds_store_swz<CKI>(dst, G * tid + e * CKI, infs);
+            for (int e = 0; e < G / CKI; ++e) lds_store_swz<CKI, SWZ>(dst, G * tid + e * CKI, infs);
         }
         if (tgt1)
             dirty1 = live;
@@ -390,7 +394,7 @@ __device__ int viterbi_gx(const float* xs, int TV, Tab& tab, int start, float* b
                     float best[CK];
 #pragma unroll
                     for (int gg = 0; gg < CK; ++gg) best[gg] = bv[HL][e] + tab.dsq(x, HL * G + e * CK + gg);
-                    lds_store_swz<CK>(dst, G * tid + e * CK, best);
+                    lds_store_swz<CK, SWZ>(dst, G * tid + e * CK, best);
                 }
                 back[t * V::ACT + tid] = (BackT)((uint32_t)HL * REP);
             };
@@ -416,7 +420,7 @@ __device__ int viterbi_gx(const float* xs, int TV, Tab& tab, int start, float* b
                     best[gg] = cost_of(m);
                     bits = (bits << K) | low_of(m);
                 }
-                lds_store_swz<CK>(dst, G * tid + e * CK, best);
+                lds_store_swz<CK, SWZ>(dst, G * tid + e * CK, best);
             }
             asm volatile("" : "+v"(bits));  // (32-bit operations above, not the stored width's)
             back[t * V::ACT + tid] = (BackT)bits;
@@ -464,7 +468,7 @@ __device__ int viterbi_gx(const float* xs, int TV, Tab& tab, int start, float* b
 #pragma unroll
                 for (int i = 0; i < CK4; ++i) infs[i] = __builtin_inff();
 #pragma unroll
-                for (int e = 0; e < G / CK4; ++e) lds_store_swz<CK4>(buf, G * tid + e * CK4, infs);
+                for (int e = 0; e < G / CK4; ++e) lds_store_swz<CK4, SWZ>(buf, G * tid + e * CK4, infs);
             }
             if (Q * tid < SPAN) {
                 // the offset through an opaque move: the addresses below are formed here, not hoisted out of the
@@ -482,7 +486,7 @@ __device__ int viterbi_gx(const float* xs, int TV, Tab& tab, int start, float* b
                 const auto common = [&](auto tc) {
                     constexpr int t = decltype(tc)::value;
                     const uint32_t idx = ((su << (K * (t + 1))) & (uint32_t)(V::NS - 1)) + (ii >> (K * (T1 - t)));
-                    c0 = c0 + tab.dsq_at(xs[t], idx);
+                    c0 = c0 + tab.dsq_at(target(t), idx);
                 };
                 static_for<0, TC + 1>(common);
 #pragma unroll
@@ -497,7 +501,7 @@ __device__ int viterbi_gx(const float* xs, int TV, Tab& tab, int start, float* b
                         constexpr int SH = K * (T1 - t);
                         constexpr int NTS = (CH >> SH) > 0 ? (CH >> SH) : 1;
                         const uint32_t idx = ((su << (K * (t + 1))) & (uint32_t)(V::NS - 1)) + (ic >> SH);
-                        const float xt = xs[t];
+                        const float xt = target(t);
                         float cn[NTS];
                         if constexpr (NTS == 1) {
                             cn[0] = cp[0] + tab.dsq_at(xt, idx);
@@ -514,7 +518,7 @@ __device__ int viterbi_gx(const float* xs, int TV, Tab& tab, int start, float* b
 #pragma unroll
                             for (int j = 0; j < NTS; ++j) cp[j] = cn[j];
                         } else {
-                            lds_store_swz<CH>(buf, rb + (int)ic, cn);
+                            lds_store_swz<CH, SWZ>(buf, rb + (int)ic, cn);
                         }
                     };
                     static_for<TC + 1, T1 + 1>(pos);
@@ -539,7 +543,7 @@ __device__ int viterbi_gx(const float* xs, int TV, Tab& tab, int start, float* b
             dirty0 = wave_live(T1);
             dirty1 = true;
             cur = 0;
-            x = xs[T1 + 1];
+            x = target(T1 + 1);
             live = wave_live(T1 + 1);
             if (act && live) {
 #pragma unroll
@@ -568,6 +572,7 @@ __device__ int viterbi_gx(const float* xs, int TV, Tab& tab, int start, float* b
         for (int t = tb; t < TV - 1; ++t) step(t, cur);
     }
     int* redi = reinterpret_cast<int*>(red + NT / 64);
+    double* redp = reinterpret_cast<double*>(red);
     constexpr bool TWOPASS = L > 12;  // (at L <= 12 a thread holds at most 16 states: one pass with the index)
     if constexpr (TWOPASS) {
         // final costs in two passes: the minimum of this thread's states (a v_min3 tree per h; a wave with no reachable
@@ -615,50 +620,47 @@ __device__ int viterbi_gx(const float* xs, int TV, Tab& tab, int start, float* b
         if ((tid & 63) == 63) redi[tid >> 6] = wbi;
     } else {
         hook();
-        // final costs, the lowest state on ties (a thread's states increase with (h, g)); a wave with no reachable
-        // member there keeps +inf
-        float bvv = __builtin_inff();
-        int bi = 0x7fffffff;
+        // final costs, the lowest state on ties: the pairs (cost, state) of this thread's members, of the wave, and (below)
+        // of the block's waves; a thread that owns none keeps (+inf, 2^31 - 1)
+        double p = cost_and(__builtin_inff(), 0x7FFFFFFFu);
         if (act && live) {
             tab.hold();
+            double q[2] = {p, p};  // (two chains)
+            // the thread's first state through an opaque move: the low words are formed here, each by one addition, and
+            // not hoisted out of the caller's loop over searches and held across it
+            uint32_t s0 = (uint32_t)(G * tid);
+            asm volatile("" : "+v"(s0));
 #pragma unroll
             for (int h = 0; h < NB; ++h)
 #pragma unroll
-                for (int g = 0; g < G; ++g) {
-                    const float c = bv[h][V::RUN ? (g >> K) : 0] + tab.dsq(x, h * G + g);
-                    if ((h == 0 && g == 0) || c < bvv) {
-                        bvv = c;
-                        bi = h * R + G * tid + g;
-                    }
-                }
+                for (int g = 0; g < G; ++g)
+                    q[g & 1] = fmin(q[g & 1], cost_and(bv[h][V::RUN ? (g >> K) : 0] + tab.dsq(x, h * G + g),
+                                                       s0 + (uint32_t)(h * R + g)));
+            p = fmin(q[0], q[1]);
         }
-        wave_argmin(bvv, bi);
-        if ((tid & 63) == 63) {
-            red[tid >> 6] = bvv;
-            redi[tid >> 6] = bi;
-        }
+        p = wave_pair_min(p);
+        if ((tid & 63) == 63) redp[tid >> 6] = p;
     }
     if (BACK_GLOBAL)
         __syncthreads();
     else
         lds_barrier();
+    buf_free();
     int pathv = 0;
     if (tid < 64) {
         // wave 0 traces back; every lane combines the waves' results, so s is uniform
-        int s = redi[0];
+        int s;
         if constexpr (TWOPASS) {
+            s = redi[0];
 #pragma unroll
             for (int wv = 1; wv < NT / 64; ++wv) s = min(s, redi[wv]);
         } else {
-            float v = red[0];
+            double m = redp[0];
 #pragma unroll
-            for (int wv = 1; wv < NT / 64; ++wv)
-                if (red[wv] < v || (red[wv] == v && redi[wv] < s)) {
-                    v = red[wv];
-                    s = redi[wv];
-                }
+            for (int wv = 1; wv < NT / 64; ++wv) m = fmin(m, redp[wv]);
+            s = (int)low_of(m);
         }
-        // no state attains the minimum only when every final cost is NaN (a NaN target: each cost of that position and
+        // a final cost of NaN (a NaN target: each cost of that position and
         // every later one is NaN; in one pass the result may then come from a thread that owns no states); the
         // reference's argmin then returns the first entry, state 0, and the traceback below stays inside the
         // back-pointers
@@ -766,7 +768,7 @@ __device__ __forceinline__ void load_block_row(double* trow, const double* __res
 //   E = T[j+c] - table64[path[c]] * S
 //   z = E U_BB^-1: z[c] = (E[c] - sum_{l<c} z[l] U[j+l][j+c]) / U[j+c][j+c], an fma chain in l (one wave)
 //   T[col] = T[col] - sum_l z[l] U[j+l][col] for col in [j+w, b1), the sum an fma chain from l = 0
-// The U operands do not depend on the row's search, so they are fetched before it and arrive while it runs.
+// The U operands do not depend on the row's path, so they are fetched before it is known and arrive under its traceback.
 
 // E (lanes c < w of wave 0, which also store the states) and the forward substitution by wave 0 given ucol[l] =
 // U[j+l][j+c] for lane c = tid % 16. Writes z to zs (LDS) and Zj.
@@ -810,7 +812,7 @@ __device__ __forceinline__ void refit_solve(UCol ucolf, double* trow, int jo, in
 }
 
 // U staged in LDS (the fused kernels with room for it): rows j..j+w of U from column j to b1, fetched by direct
-// global->LDS loads before the search (wave v of NT/64 takes rows v, v + NT/64, ...; four 64-dword pieces per
+// global->LDS loads under the search's traceback, where the minima lay (wave v of NT/64 takes rows v, v + NT/64, ...; four 64-dword pieces per
 // row), urows[l][c] = U[j+l][j+c]. No registers are held across the search.
 template <int NT, int LAZY>
 __device__ __forceinline__ void refit_fetch_lds(double (*urows)[LAZY], const double* __restrict__ U, int64_t ldU,

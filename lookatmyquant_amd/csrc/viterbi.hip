@@ -3,9 +3,14 @@
 #include "trellis.h"
 
 #define LAMQ_TV_LDS 32  // longest standalone path whose back-pointers stay in LDS
-#define LAMQ_TV_BLK 24  // longest search of the fused block (width + look): with lazy <= 128 the block kernel's
-                        // LDS stays under 40 KB, four workgroups per CU
+#define LAMQ_TV_BLK 24  // longest search of the fused block (width + look)
 #define LAMQ_LAZY_MAX 128
+// Workgroups of the fused block a CU holds (four waves each, one per SIMD). A row's search alternates steps that fill
+// the vector unit with stretches of latency (a barrier and an LDS round trip per step, the traceback, the refit's chain),
+// which only other rows cover: 6,144 x 2,560 at L = 12, 1 to 4 bits: 12.6 ms with four, 11.2 with five, 10.5 with six.
+// Six is what fits: 23.8 KB of LDS (the step's rows of U take the minima's place, which are free by then, instead of
+// 16 KB of their own: four fitted) and 80 registers.
+#define LAMQ_BLK_WAVES 6
 
 // ------------------------------------------------------------------------------------------------
 // viterbi_rows: one workgroup per row (opgraph/codes.py:151-181).
@@ -20,14 +25,14 @@ __global__ __launch_bounds__(LAMQ_NT) void viterbi_rows_kernel(const float* __re
     using V = VX<L, K, LAMQ_NT>;
     __shared__ __align__(16) float buf[2 * V::R];
     __shared__ uint8_t back_lds[BACK_GLOBAL ? 1 : (LAMQ_TV_LDS - 1) * V::ACT];
-    __shared__ float red[2 * (LAMQ_NT / 64)];
+    __shared__ __align__(8) float red[2 * (LAMQ_NT / 64)];
     const int64_t row = blockIdx.x;
     const int tid = threadIdx.x;
     TabF32<V> tab;
     if (tid < V::ACT) tab.load(C, tid);
     uint8_t* back = BACK_GLOBAL ? back_ws + row * (int64_t)(T - 1) * V::ACT : back_lds;
     const int st = start ? start[row] : -1;
-    viterbi_gx<L, K, LAMQ_NT, true, BACK_GLOBAL>(x + row * ldx, T, tab, st, buf, back, states + row * lds, red);
+    viterbi_gx<L, K, LAMQ_NT, true, BACK_GLOBAL, false, true>(x + row * ldx, T, tab, st, buf, back, states + row * lds, red);
 }
 
 template <int L, int K>
@@ -236,20 +241,23 @@ static bool wide_lk(int L, int k)
 //           beyond b1 still lack this block's trailing update (they are read as they stand)
 //   path  = viterbi(xs, start = state)[:w];  state = path[w-1]
 //   then the refit of trellis.h (E, z = E U_BB^-1, the in-block update of the columns up to b1).
-// The block's columns of T live in LDS for the whole block; T in HBM is not written (the settled
+// The rows of U are fetched under the traceback. The block's columns of T live in LDS for the whole block; T in HBM is not written (the settled
 // values are table64[states] * S; columns >= b1 get the trailing update from Z afterwards).
 // ------------------------------------------------------------------------------------------------
 template <int L, int K>
 struct alignas(16) BlkSmem {
     using V = VX<L, K, LAMQ_NT>;
-    float buf[2 * V::R];
+    // the search's minima; once its forward pass is done, the step's rows of U
+    union {
+        float buf[2 * V::R];
+        double urows[LAMQ_WMAX][LAMQ_LAZY_MAX];
+    };
     uint8_t back[(LAMQ_TV_BLK - 1) * V::ACT];
     double trow[LAMQ_LAZY_MAX + LAMQ_TV_BLK];
-    double urows[LAMQ_WMAX][LAMQ_LAZY_MAX];
     double zs[LAMQ_WMAX];
     float xs[LAMQ_TV_BLK];
     int path[LAMQ_TV_BLK];
-    float red[2 * (LAMQ_NT / 64)];
+    alignas(8) float red[2 * (LAMQ_NT / 64)];
 };
 
 // One row's lazy block [b0, b1): `row` indexes T, S, state, states and Z.
@@ -279,10 +287,11 @@ __device__ __forceinline__ void trellis_block_row(BlkSmem<L, K>& sm, int64_t row
         const int TV = w + a;
         const int jo = (int)(j - b0);
         const int nc = (int)(b1 - j - w);
-        refit_fetch_lds<LAMQ_NT, LAMQ_LAZY_MAX>(sm.urows, U, ldU, j, w, b1);
-        if (tid < TV) sm.xs[tid] = (float)(sm.trow[jo + tid] / Sr);
+        if (tid < TV) sm.xs[tid] = search_target((float)(sm.trow[jo + tid] / Sr));
         lds_barrier();
-        const int pv = viterbi_gx<L, K, LAMQ_NT, true, false, true>(sm.xs, TV, tab, st, sm.buf, sm.back, sm.path, sm.red);
+        const int pv = viterbi_gx<L, K, LAMQ_NT, true, false, true>(
+            sm.xs, TV, tab, st, sm.buf, sm.back, sm.path, sm.red, NoHook(),
+            [&]() { refit_fetch_lds<LAMQ_NT, LAMQ_LAZY_MAX>(sm.urows, U, ldU, j, w, b1); });
         refit_apply_lds<LAMQ_NT, LAMQ_LAZY_MAX>(sm.urows, sm.trow, jo, w, nc, pv, table64, Sr, states + row * lds + j,
                                                 Z + row * ldZ + jo, sm.zs);
         st = sm.path[w - 1];
@@ -291,7 +300,7 @@ __device__ __forceinline__ void trellis_block_row(BlkSmem<L, K>& sm, int64_t row
 }
 
 template <int L, int K>
-__global__ __launch_bounds__(LAMQ_NT, 4) void ldlq_trellis_block_kernel(
+__global__ __launch_bounds__(LAMQ_NT, LAMQ_BLK_WAVES) void ldlq_trellis_block_kernel(
     const double* __restrict__ T, int64_t n, int64_t ldT, const double* __restrict__ U, int64_t ldU,
     const double* __restrict__ S, const double* __restrict__ table64, const float* __restrict__ table32,
     int64_t b0, int64_t b1, int width, int look, int32_t* __restrict__ state, int32_t* __restrict__ states,
@@ -337,7 +346,7 @@ extern "C" int lamq_ldlq_trellis_block(double* T, int64_t m, int64_t n, int64_t 
 // tail of partly idle CUs (four 256-thread rows per CU, so ceil(rows / 1024) rounds), which one launch over all their
 // rows does not have. Workgroup b takes row b of the concatenated groups (in the table's order), finds its group (a
 // uniform scan of at most LAMQ_TRELLIS_MAX_GROUPS entries) and runs that width's block in that width's LDS layout
-// over one shared array (the widest layout's size: four workgroups per CU as for each width alone).
+// over one shared array (the widest layout's size: as many workgroups per CU as for each width alone).
 #define LAMQ_GROUPS_L 12
 struct BlkGroup {
     int64_t r0, rows;
@@ -361,12 +370,12 @@ constexpr int blk_groups_smem_bytes()
 }
 
 template <int L>
-__global__ __launch_bounds__(LAMQ_NT, 4) void ldlq_trellis_groups_kernel(
+__global__ __launch_bounds__(LAMQ_NT, LAMQ_BLK_WAVES) void ldlq_trellis_groups_kernel(
     const double* __restrict__ T, int64_t n, int64_t ldT, const double* __restrict__ U, int64_t ldU,
     const double* __restrict__ S, int64_t b0, int64_t b1, int width, int look, int32_t* __restrict__ state,
     int32_t* __restrict__ states, int64_t lds, double* __restrict__ Z, int64_t ldZ, int pre, BlkGroups groups)
 {
-    static_assert(blk_groups_smem_bytes<L>() * 4 <= 160 * 1024, "four workgroups per CU");
+    static_assert(blk_groups_smem_bytes<L>() * 6 <= 160 * 1024, "six workgroups per CU");
     __shared__ __align__(16) uint8_t raw[blk_groups_smem_bytes<L>()];
     int64_t b = blockIdx.x;
     int i = 0;

@@ -243,7 +243,7 @@ __global__ __launch_bounds__(BIG_NT) void viterbi_rows_gx_kernel(const float* __
     TabF16<V> tab;
     tab.load(table16, threadIdx.x);
     uint32_t* back = BACK_GLOBAL ? back_ws + row * (int64_t)(T - 1) * BIG_NT : back_lds;
-    viterbi_gx<L, K, BIG_NT, DBL, BACK_GLOBAL>(x + row * ldx, T, tab, start ? start[row] : -1, buf, back,
+    viterbi_gx<L, K, BIG_NT, DBL, BACK_GLOBAL, false, true>(x + row * ldx, T, tab, start ? start[row] : -1, buf, back,
                                              states + row * lds, red);
 }
 
@@ -447,7 +447,7 @@ __device__ __forceinline__ void gx_block_row(GxSmem<L, K, BG>& sm, int64_t row, 
         const int TV = w + a;
         const int jo = (int)(j - b0);
         const int nc = (int)(b1 - j - w);
-        if (tid < TV) xs[tid] = (float)(trow[jo + tid] / Sr);
+        if (tid < TV) xs[tid] = search_target((float)(trow[jo + tid] / Sr));
         lds_barrier();
         // the refit's U operands are fetched when the forward pass ends, under the final argmin and the traceback
         RefitRegs<4> ops;

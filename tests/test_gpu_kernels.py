@@ -120,6 +120,23 @@ def test_ldlq_trellis_L16_ties_match_oracle(E, k):
     assert np.array_equal(st, O.ldlq_trellis(X, U, S, tab, 16, k))
 
 
+@pytest.mark.parametrize("L,k", [(12, 1), (12, 2), (12, 3), (12, 4), (9, 2), (16, 2), (16, 3), (16, 4)])
+def test_viterbi_nan_and_infinite_targets_match_oracle(E, L, k):
+    """A NaN of either sign, or an infinity, among the last targets: from there on every path cost is NaN (or +inf), every
+    group keeps its lowest h and the path ends in state 0, as the oracle's strict comparisons leave it."""
+    from lookatmyquant_amd.tables import quantile_table
+
+    tab = quantile_table(L, 0)
+    rng = np.random.default_rng(900 + 10 * L + k)
+    x = rng.standard_normal((5, 24)).astype(np.float32)
+    bad = np.array([0x7FC00000, 0xFFC00000, 0xFFFFFFFF, 0x7F800000, 0xFF800000], dtype=np.uint32).view(np.float32)
+    x[np.arange(5), [20, 20, 22, 20, 23]] = bad
+    st = rng.integers(0, 1 << L, 5)
+    say(f"viterbi L={L} k={k}, NaN and infinite targets")
+    got = E.viterbi_rows(cuda(x), cuda(tab.astype(np.float32)), L, k, start=cuda(st, torch.int32)).cpu().numpy()
+    assert np.array_equal(got, O.viterbi(x, tab, L, k, start=st))
+
+
 def test_viterbi_L16_long_paths_use_workspace(E):
     from lookatmyquant_amd.tables import quantile_table
 
