@@ -48,40 +48,45 @@ __device__ __forceinline__ int64_t xcd_remap(int64_t b, int64_t G)
     return x < extra ? x * (q + 1) + r : extra * (q + 1) + (x - extra) * q + r;
 }
 
-// LDS float index -> bank-spread index: the 16-byte chunk index (x >> 2) has its low two bits xor'ed with bits
-// 4-5 of itself, a bijection within every 64 floats. Writes of consecutive threads at a stride of 16 floats then
-// fall on 16 different 16-byte bank groups, and reads of consecutive 16-byte chunks stay conflict-free.
-__device__ __forceinline__ int swz(int x) { return x ^ (((x >> 6) & 3) << 2); }
+// LDS float index -> bank-spread index: the 16-byte chunk index (x >> 2) has its low bits xor'ed with the bits of itself
+// from bit 4 up that MASK selects, a bijection within every 64 floats. Threads that each hold 4 (MASK + 1) consecutive
+// floats then write their j-th chunks to 16 different 16-byte bank groups, 16 threads at a time, and reads of
+// consecutive chunks (or of runs of a power of two of them) stay conflict-free. MASK 0: the index itself.
+template <int MASK = 3>
+__device__ __forceinline__ int swz(int x)
+{
+    return x ^ (((x >> 6) & MASK) << 2);
+}
 
-// N floats at logical index x (x a multiple of min(N, 4)), chunk by chunk through swz (SWZ false: at x itself).
-template <int N, bool SWZ = true>
+// N floats at logical index x (x a multiple of min(N, 4)), chunk by chunk through swz.
+template <int N, int MASK = 3>
 __device__ __forceinline__ void lds_load_swz(const float* __restrict__ base, int x, float (&dst)[N])
 {
     if constexpr (N >= 4) {
 #pragma unroll
         for (int i = 0; i < N; i += 4) {
-            float4 v = *reinterpret_cast<const float4*>(base + (SWZ ? swz(x + i) : x + i));
+            float4 v = *reinterpret_cast<const float4*>(base + swz<MASK>(x + i));
             dst[i] = v.x; dst[i + 1] = v.y; dst[i + 2] = v.z; dst[i + 3] = v.w;
         }
     } else if constexpr (N == 2) {
-        float2 v = *reinterpret_cast<const float2*>(base + (SWZ ? swz(x) : x));
+        float2 v = *reinterpret_cast<const float2*>(base + swz<MASK>(x));
         dst[0] = v.x; dst[1] = v.y;
     } else {
-        dst[0] = base[SWZ ? swz(x) : x];
+        dst[0] = base[swz<MASK>(x)];
     }
 }
 
-template <int N, bool SWZ = true>
+template <int N, int MASK = 3>
 __device__ __forceinline__ void lds_store_swz(float* __restrict__ base, int x, const float (&src)[N])
 {
     if constexpr (N >= 4) {
 #pragma unroll
         for (int i = 0; i < N; i += 4)
-            *reinterpret_cast<float4*>(base + (SWZ ? swz(x + i) : x + i)) = make_float4(src[i], src[i + 1], src[i + 2], src[i + 3]);
+            *reinterpret_cast<float4*>(base + swz<MASK>(x + i)) = make_float4(src[i], src[i + 1], src[i + 2], src[i + 3]);
     } else if constexpr (N == 2) {
-        *reinterpret_cast<float2*>(base + (SWZ ? swz(x) : x)) = make_float2(src[0], src[1]);
+        *reinterpret_cast<float2*>(base + swz<MASK>(x)) = make_float2(src[0], src[1]);
     } else {
-        base[SWZ ? swz(x) : x] = src[0];
+        base[swz<MASK>(x)] = src[0];
     }
 }
 

@@ -32,10 +32,18 @@ struct VX {
     // h*(R >> K) + M*t. G < NB: one entry per h, (h*R + G*t) >> K, shared by NB/G neighbouring threads.
     static constexpr bool RUN = G >= NB;
     static constexpr int M = RUN ? G / NB : 1;
-    // Up to four groups a thread, its minima are one 16-byte chunk beside its neighbours' and neither the stores nor the
-    // reads meet bank conflicts; a thread of more stores chunks at a stride, spread by swz. Without it every entry a
-    // thread reads lies at one index plus a constant (one address register, not NB).
-    static constexpr bool SWZ = G > 4;
+    // The swizzle of the minima (common.h, swz): a thread's G floats are G / 4 chunks. Up to four groups a thread they are
+    // one chunk beside its neighbours' and need none; without it (or wherever R >> K is a multiple of 64 (SWZ + 1))
+    // every entry a thread reads lies at one index plus a constant (one address register, not NB).
+    static constexpr int SWZ = G <= 4 ? 0 : (G / 4 < 16 ? G / 4 : 16) - 1;
+    // Back-pointer words of `bits` bits: group_word groups each (a power of two), step_words of them a step.
+    static constexpr int group_word(int bits)
+    {
+        int g = G;
+        while (g * K > bits) g /= 2;
+        return g;
+    }
+    static constexpr int step_words(int bits) { return ACT * (G / group_word(bits)); }
 };
 
 // s_waitcnt lgkmcnt(0) + s_barrier: orders this workgroup's LDS traffic without waiting for its
@@ -193,6 +201,50 @@ __device__ __forceinline__ double pair_min(const float (&c)[N], const LowWords<N
     return m[0];
 }
 
+// fp16 values widened to float32 in registers: twice the registers, and x - C is a 2-clock subtraction where v_fma_mix_f32
+// takes 4 (2,560 x 256 at L = 16, 1,024 threads of halves -> 512 of these: k = 2 6.35 -> 5.78 ms, k = 3 7.03 -> 5.74,
+// k = 4 7.27 -> 6.25).
+template <class V>
+struct TabF16Wide {
+    float v[V::SPT];
+    const uint16_t* src;
+    __device__ __forceinline__ void load(const uint16_t* __restrict__ C16, int t)
+    {
+        src = C16;
+#pragma unroll
+        for (int h = 0; h < V::NB; ++h)
+#pragma unroll
+            for (int g = 0; g < V::G; g += 2) {
+                const uint32_t w = *reinterpret_cast<const uint32_t*>(C16 + h * V::R + V::G * t + g);
+                v[h * V::G + g] = h2f_lo(w);
+                v[h * V::G + g + 1] = h2f_hi(w);
+            }
+    }
+    // keeps the widened values in registers (the compiler would keep the halves and convert them in every step)
+    __device__ __forceinline__ void hold()
+    {
+#pragma unroll
+        for (int i = 0; i < V::SPT; ++i) asm volatile("" : "+v"(v[i]));
+    }
+    __device__ __forceinline__ float dsq(float x, int i) const
+    {
+        const float d = x - v[i];
+        return d * d;
+    }
+    __device__ __forceinline__ float dsq_at(float x, uint32_t s) const
+    {
+        const float d = xmc_lo(x, (uint32_t)src[s]);
+        return d * d;
+    }
+    __device__ __forceinline__ void dsq_at2(float x, uint32_t s, float& q0, float& q1) const
+    {
+        const uint32_t w = *reinterpret_cast<const uint32_t*>(src + s);
+        const float d0 = xmc_lo(x, w), d1 = xmc_hi(x, w);
+        q0 = d0 * d0;
+        q1 = d1 * d1;
+    }
+};
+
 // f(IntC<v>{}) for the uniform v in [I, N): a chain of scalar branches, so that f indexes registers statically
 template <int I>
 struct IntC {
@@ -278,8 +330,8 @@ __device__ __forceinline__ int wave_imin(int v)
 //   xs: TV float32 targets (LDS or global), through search_target already or, with RAWX, as they come. start < 0 leaves
 //   the first state free, else only the states (start << K | b) & (2^L - 1) may begin (codes.py:164-167). buf: DBL ? 2R
 //   : R floats of LDS (with one buffer each step takes a second barrier, between the reads of the old minima and the
-//   writes of the new). back: (TV-1) * ACT entries (LDS or global), entry t*ACT + owner holding the winning h of each of
-//   the owner's groups for the step that produced B_{t+1}. red: 2*(NT/64) words of LDS, 8-byte aligned.
+//   writes of the new). back: (TV-1) * WPS words (LDS or global), word t*WPS + r/GW holding the winning h of group r (and
+//   of the GW - 1 others of its word) for the step that produced B_{t+1}. red: 2*(NT/64) words of LDS, 8-byte aligned.
 //   Final state: the lowest among the minimal costs (codes.py:173); traceback codes.py:176-179.
 // hook() runs once the forward pass is done (the caller's chance to issue loads that the end of the final argmin and
 // the traceback then cover; at L > 12 after the argmin's two passes over the states). BACK_GLOBAL: back-pointers in
@@ -293,20 +345,24 @@ __device__ int viterbi_gx(const float* xs, int TV, Tab& tab, int start, float* b
 {
     using V = VX<L, K, NT>;
     constexpr int G = V::G, NB = V::NB, M = V::M, R = V::R;
-    static_assert(G * K <= 8 * (int)sizeof(BackT), "one back-pointer entry per thread and step");
+    // back-pointer words: GW groups each (a power of two), W words a thread and step, word r / GW holding group r's h
+    constexpr int GW = V::group_word(8 * (int)sizeof(BackT));
+    constexpr int W = G / GW;
+    constexpr int WPS = V::step_words(8 * (int)sizeof(BackT));
     const int tid = threadIdx.x;
     // every thread owns groups when there are at least NT of them (the kernels launch exactly NT threads): a
     // compile-time true then, and the step loop carries no exec-mask branches
     const bool act = V::ACT >= NT || tid < V::ACT;
+    // groups stored together: those sharing one B entry per h, and four at least
+    constexpr int CK = V::RUN ? (NB < 4 && G >= 4 ? 4 : NB) : G;
     int ent[NB];
 #pragma unroll
     for (int h = 0; h < NB; ++h) ent[h] = V::RUN ? h * (R >> K) + M * tid : (h * R + G * tid) >> K;
     float bv[NB][M];
-    // ent[h] = ent[0] + h (R >> K), if R >> K entries hold whole neighbourhoods of threads sharing one; where that stride
-    // is a multiple of 256 the swizzle keeps it too (swz(x + 256 i) = swz(x) + 256 i): every h then reads at one index plus
-    // a constant offset (one register, not NB)
-    constexpr bool SWZ = V::SWZ;
-    constexpr bool EOFF = (R >> K) << K == R && (!SWZ || (R >> K) % 256 == 0);
+    // ent[h] = ent[0] + h (R >> K) where R is a multiple of 2^K; a stride the swizzle keeps (swz(x + d) = swz(x) + d)
+    // then makes one swizzled index serve every h
+    constexpr int SWZ = V::SWZ;
+    constexpr bool EOFF = (R >> K) << K == R && (SWZ == 0 || (R >> K) % (64 * (SWZ + 1)) == 0);
     const auto load_minima = [&](const float* b, int h) {
         if constexpr (EOFF)
             lds_load_swz<M, SWZ>(b + h * (R >> K), ent[0], bv[h]);
@@ -322,7 +378,9 @@ __device__ int viterbi_gx(const float* xs, int TV, Tab& tab, int start, float* b
 #pragma unroll
             for (int e = 0; e < M; ++e) bv[h][e] = (rs < 0 || d == h * (R >> K) + e) ? 0.0f : __builtin_inff();
     };
-    const LowWords<NB> lo;
+    // (a thread of many states has no registers to spare for sixteen of them: two halves of eight)
+    constexpr int NLO = NB == 16 && V::SPT > 64 ? 8 : NB;
+    const LowWords<NLO> lo;
     const auto target = [&](int t) { return RAWX ? search_target(xs[t]) : xs[t]; };
     int cur = 0;
     float x = target(0);
@@ -338,7 +396,7 @@ __device__ int viterbi_gx(const float* xs, int TV, Tab& tab, int start, float* b
     constexpr bool SKIP = L >= 16;
     constexpr uint32_t REP = [] {  // hl in every group's K-bit field of a back-pointer word
         uint32_t r = 0;
-        for (int g = 0; g < G; ++g) r |= 1u << (g * K);
+        for (int g = 0; g < GW; ++g) r |= 1u << (g * K);
         return r;
     }();
     const int wv = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -371,7 +429,7 @@ __device__ int viterbi_gx(const float* xs, int TV, Tab& tab, int start, float* b
         const bool one_h = SKIP && st0 >= 0 && K * (t + 1) <= L - K;
         const bool tgt1 = DBL && cur == 0;  // the buffer this step writes: cur ^ 1 (DBL), else the only one
         if (act && !live && (tgt1 ? dirty1 : dirty0)) {
-            constexpr int CKI = V::RUN ? NB : G;
+            constexpr int CKI = CK;
             float* dst = buf + (DBL ? (cur ^ 1) * R : 0);
             float infs[CKI];
 #pragma unroll
@@ -388,42 +446,60 @@ __device__ int viterbi_gx(const float* xs, int TV, Tab& tab, int start, float* b
             float* dst = buf + (DBL ? (cur ^ 1) * R : 0);
             auto step1 = [&](auto hc) {
                 constexpr int HL = decltype(hc)::value;
-                constexpr int CK = V::RUN ? NB : G;
-#pragma unroll
-                for (int e = 0; e < G / CK; ++e) {
+                const auto chunk1 = [&](auto ec) {
+                    constexpr int e = decltype(ec)::value;
                     float best[CK];
 #pragma unroll
-                    for (int gg = 0; gg < CK; ++gg) best[gg] = bv[HL][e] + tab.dsq(x, HL * G + e * CK + gg);
+                    for (int gg = 0; gg < CK; ++gg) best[gg] = bv[HL][V::RUN ? (e * CK + gg) >> K : 0] + tab.dsq(x, HL * G + e * CK + gg);
                     lds_store_swz<CK, SWZ>(dst, G * tid + e * CK, best);
-                }
-                back[t * V::ACT + tid] = (BackT)((uint32_t)HL * REP);
+                };
+                static_for<0, G / CK>(chunk1);
+#pragma unroll
+                for (int w = 0; w < W; ++w) back[t * WPS + tid * W + w] = (BackT)((uint32_t)HL * REP);
+                // a different end for each slab: the compiler would merge the branches and index the registers by slab
+                asm volatile("; slab %0" ::"n"(HL));
             };
             uniform_switch<0, NB>(base >> (L - K), step1);
         }
         if (act && live && !one_h) {
             tab.hold();
-            uint32_t bits = 0;
+            uint32_t bits = 0, words[W];
             float* dst = buf + (DBL ? (cur ^ 1) * R : 0);
-            // groups in chunks of CK sharing one B entry per h (RUN) or all of them, from the last to the first (the
-            // winning h are shifted in, group 0's last); each chunk stored when done
-            constexpr int CK = V::RUN ? NB : G;
-#pragma unroll
-            for (int e = G / CK - 1; e >= 0; --e) {
+            // groups in chunks of CK, from the last to the first (the winning h are shifted in, group 0's last); each chunk
+            // stored when done
+            const auto chunk = [&](auto ec) {  // (a template per chunk: as a loop of many it is not unrolled)
+                constexpr int e = G / CK - 1 - decltype(ec)::value;
                 float best[CK];
 #pragma unroll
                 for (int gg = CK - 1; gg >= 0; --gg) {
                     const int g = e * CK + gg;
-                    float c[NB];
+                    float c[NLO];
 #pragma unroll
-                    for (int h = 0; h < NB; ++h) c[h] = bv[h][e] + tab.dsq(x, h * G + g);
-                    const double m = pair_min<NB>(c, lo);
+                    for (int h = 0; h < NLO; ++h) c[h] = bv[h][V::RUN ? (g >> K) : 0] + tab.dsq(x, h * G + g);
+                    double m = pair_min<NLO>(c, lo);
+                    if constexpr (NLO < NB) {
+                        __builtin_amdgcn_sched_barrier(0);  // (the halves in turn: together they take copies of lo)
+#pragma unroll
+                        for (int h = 0; h < NLO; ++h) c[h] = bv[NLO + h][V::RUN ? (g >> K) : 0] + tab.dsq(x, (NLO + h) * G + g);
+                        const double m2 = pair_min<NLO>(c, lo);
+                        m = fmin(m, cost_and(cost_of(m2), low_of(m2) | (uint32_t)NLO));
+                        __builtin_amdgcn_sched_barrier(0);
+                    }
                     best[gg] = cost_of(m);
                     bits = (bits << K) | low_of(m);
+                    if (g % GW == 0) {
+                        words[g / GW] = bits;
+                        bits = 0;
+                    }
                 }
                 lds_store_swz<CK, SWZ>(dst, G * tid + e * CK, best);
+            };
+            static_for<0, G / CK>(chunk);
+#pragma unroll
+            for (int w = 0; w < W; ++w) {
+                asm volatile("" : "+v"(words[w]));  // (32-bit operations above, not the stored width's)
+                back[t * WPS + tid * W + w] = (BackT)words[w];
             }
-            asm volatile("" : "+v"(bits));  // (32-bit operations above, not the stored width's)
-            back[t * V::ACT + tid] = (BackT)bits;
         }
         lds_barrier();
         cur ^= 1;
@@ -529,14 +605,17 @@ __device__ int viterbi_gx(const float* xs, int TV, Tab& tab, int start, float* b
             // over searches and held across it)
             int to = tid;
             asm volatile("" : "+v"(to));
-            BackT* const bw = back + to;
+            BackT* const bw = back + to * W;
             const auto words = [&](auto tc) {
                 constexpr int t = decltype(tc)::value;
                 constexpr int span = 1 << (K * (t + 1));
                 constexpr int no = span >= G ? span / G : 1;
                 const uint32_t base = (su << (K * (t + 1))) & (uint32_t)(V::NS - 1);
                 const int olo = (int)(base & (uint32_t)(R - 1)) / G;
-                if (tid >= olo && tid < olo + no) bw[t * V::ACT] = (BackT)((base >> (L - K)) * REP);
+                if (tid >= olo && tid < olo + no) {
+#pragma unroll
+                    for (int w = 0; w < W; ++w) bw[t * WPS + w] = (BackT)((base >> (L - K)) * REP);
+                }
             };
             static_for<0, T1 + 1>(words);
             lds_barrier();
@@ -583,14 +662,15 @@ __device__ int viterbi_gx(const float* xs, int TV, Tab& tab, int start, float* b
         float mine = __builtin_inff();
         if (act && live) {
             tab.hold();
-#pragma unroll
-            for (int h = 0; h < NB; ++h) {
+            const auto least = [&](auto hc) {
+                constexpr int h = decltype(hc)::value;
                 float m = __builtin_inff();
 #pragma unroll
                 for (int g = 0; g < G; ++g) m = fminf(m, bv[h][V::RUN ? (g >> K) : 0] + tab.dsq(x, h * G + g));
                 if constexpr (KEEPH) mh[h] = m;
                 mine = fminf(mine, m);
-            }
+            };
+            static_for<0, NB>(least);
         }
         const float wmin = wave_min(mine);
         if ((tid & 63) == 63) red[tid >> 6] = wmin;
@@ -601,19 +681,22 @@ __device__ int viterbi_gx(const float* xs, int TV, Tab& tab, int start, float* b
         int bi = 0x7fffffff;
         if (act && live && mine == mb) {
             tab.hold();
-            // x through an opaque move: the costs are formed again here, not kept from the first pass (64 registers)
+            // x and the thread's first group through opaque moves: the costs are formed again here, not kept from the
+            // first pass, and the states here, not hoisted out of the caller's loop (a register each)
             float xo = x;
-            asm volatile("" : "+v"(xo));
-#pragma unroll
-            for (int h = 0; h < NB; ++h) {
+            int g0 = G * tid;
+            asm volatile("" : "+v"(xo), "+v"(g0));
+            const auto find = [&](auto hc) {
+                constexpr int h = decltype(hc)::value;
                 if (bi == 0x7fffffff && (!KEEPH || mh[KEEPH ? h : 0] == mb)) {
 #pragma unroll
                     for (int g = 0; g < G; ++g) {
                         const float c = bv[h][V::RUN ? (g >> K) : 0] + tab.dsq(xo, h * G + g);
-                        bi = (c == mb && bi == 0x7fffffff) ? h * R + G * tid + g : bi;
+                        bi = (c == mb && bi == 0x7fffffff) ? h * R + g0 + g : bi;
                     }
                 }
-            }
+            };
+            static_for<0, NB>(find);
         }
         hook();  // (after both passes, whose registers the caller's loads would otherwise share)
         const int wbi = wave_imin(bi);
@@ -677,13 +760,13 @@ __device__ int viterbi_gx(const float* xs, int TV, Tab& tab, int start, float* b
         // the words of the groups step t-1 continues from (one per h that step t may pick); with D = 3, lanes
         // NB+1 .. NB+NB^2 those of step t-2 (one per pair of picks). Then the picks resolve through readlane.
         constexpr int D = (1 + NB + NB * NB <= 64) ? 3 : 2;
-        constexpr int LG = __builtin_ctz(G);
+        constexpr int LG = __builtin_ctz(GW);
         const int lane = tid;
         const int level = lane == 0 ? 0 : (lane <= NB ? 1 : ((D == 3 && lane <= NB + NB * NB) ? 2 : 0));
         const uint32_t sp1 = (uint32_t)(level == 1 ? lane - 1 : (level == 2 ? (lane - 1 - NB) / NB : 0)) * R;
         const uint32_t sp2 = (uint32_t)(level == 2 ? (lane - 1 - NB) % NB : 0) * R;
         const auto pick = [&](uint32_t word, uint32_t r) {  // the state before r's group at that step
-            return r + ((word >> ((r & (G - 1)) * K)) & (uint32_t)(NB - 1)) * (uint32_t)R;
+            return r + ((word >> ((r & (GW - 1)) * K)) & (uint32_t)(NB - 1)) * (uint32_t)R;
         };
         int t = TV - 1;
         for (; t >= D; t -= D) {
@@ -691,7 +774,7 @@ __device__ int viterbi_gx(const float* xs, int TV, Tab& tab, int start, float* b
             uint32_t grp = r;
             if (level >= 1) grp = (grp + sp1) >> K;
             if (level >= 2) grp = (grp + sp2) >> K;
-            const uint32_t wd = (uint32_t)back[(t - 1 - level) * V::ACT + (grp >> LG)];
+            const uint32_t wd = (uint32_t)back[(t - 1 - level) * WPS + (grp >> LG)];
             const uint32_t s1 = pick((uint32_t)__builtin_amdgcn_readfirstlane((int)wd), r);
             const uint32_t h1 = s1 >> (L - K);
             const uint32_t s2 = pick((uint32_t)__builtin_amdgcn_readlane((int)wd, 1 + h1), s1 >> K);
@@ -708,7 +791,7 @@ __device__ int viterbi_gx(const float* xs, int TV, Tab& tab, int start, float* b
         }
         for (; t >= 1; --t) {
             const uint32_t r = (uint32_t)s >> K;
-            s = (int)pick((uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)back[(t - 1) * V::ACT + (r >> LG)]), r);
+            s = (int)pick((uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)back[(t - 1) * WPS + (r >> LG)]), r);
             emit(t - 1, s);
         }
         if (PATHREG && tid < TV) path[tid] = pathv;

@@ -1,7 +1,7 @@
 // Trellis search with 2^13 .. 2^16 states (the 16-bit-state configurations), standalone and fused into the
-// row-trellis LDLQ block. One 1024-thread workgroup per row; the state values are packed fp16 in VGPRs (the
-// kernels take tables whose values fp16 holds exactly, as the 16-bit configurations' Gaussian-quantile table;
-// x - C is then exact in float32). Back-pointers are one 32-bit word per thread and step (G*k <= 32 bits), in LDS.
+// row-trellis LDLQ block. One workgroup per row and CU (gx_nt threads; 1024 in the quarter-window search below); the
+// kernels take tables whose values fp16 holds exactly (as the 16-bit configurations' Gaussian-quantile table) and keep
+// the state values in VGPRs. Back-pointers are 32-bit words, at most 1024 a step, in LDS or in a workspace.
 //
 // Up to 2^14 groups (every configuration but L = 16, k = 1) the search is trellis.h's: only the group minima
 // (at most 64 KB) pass through LDS each step.
@@ -19,9 +19,21 @@
 // hence the same float32 value.
 #include "trellis.h"
 
+#include <type_traits>
+
 #define BIG_NT 1024
 #define BIG_TV 24       // longest fused search: width + look
 #define BIG_LAZY 128
+#define BIG_BACK_WORDS ((BIG_TV - 1) * BIG_NT)  // back-pointer words of a row in the workspace
+// Threads of a row in the minima-exchange kernels, and the form of the state values in registers: widened to float32
+// (TabF16Wide). At 16 bits those are 128 values a thread of eight waves, which have 256 registers each; sixteen waves of
+// 64 values have 128, too few beside the group minima. k = 1, whose 64 minima a thread would not fit beside them in the
+// kernel of all widths (alone: 5.64 -> 5.20 ms at 2,560 x 256; in a row plan's launch its spills cost more), keeps halves.
+template <int L>
+constexpr int gx_nt() { return L >= 16 ? 512 : BIG_NT; }
+template <int L, int K>
+using GxTab =
+    std::conditional_t<L == 16 && K == 1, TabF16<VX<L, K, gx_nt<L>()>>, TabF16Wide<VX<L, K, gx_nt<L>()>>>;
 #define BIG_GX_MAX_R 16384  // most groups of the minima-exchange search (64 KB of LDS)
 // most groups whose back-pointers the merged row-group kernel keeps in LDS; above, they go to the workspace, and the
 // LDS they leave holds a second minima buffer (one barrier a step instead of two)
@@ -228,23 +240,24 @@ __global__ __launch_bounds__(BIG_NT) void viterbi_rows_big_kernel(const float* _
 
 // minima-exchange search (trellis.h), for up to BIG_GX_MAX_R groups
 template <int L, int K, bool BACK_GLOBAL>
-__global__ __launch_bounds__(BIG_NT) void viterbi_rows_gx_kernel(const float* __restrict__ x, int T, int64_t ldx,
+__global__ __launch_bounds__(gx_nt<L>(), gx_nt<L>() / 256) void viterbi_rows_gx_kernel(const float* __restrict__ x, int T, int64_t ldx,
                                                                  const uint16_t* __restrict__ table16,
                                                                  const int32_t* __restrict__ start,
                                                                  int32_t* __restrict__ states, int64_t lds,
                                                                  uint32_t* __restrict__ back_ws)
 {
-    using V = VX<L, K, BIG_NT>;
+    constexpr int NT = gx_nt<L>();
+    using V = VX<L, K, NT>;
     constexpr bool DBL = V::R <= 4096;
     __shared__ __align__(16) float buf[(DBL ? 2 : 1) * V::R];
-    __shared__ uint32_t back_lds[BACK_GLOBAL ? 1 : (BIG_TV - 1) * V::ACT];
-    __shared__ float red[2 * (BIG_NT / 64)];
+    __shared__ uint32_t back_lds[BACK_GLOBAL ? 1 : (BIG_TV - 1) * V::step_words(32)];
+    __shared__ float red[2 * (NT / 64)];
     const int64_t row = blockIdx.x;
-    TabF16<V> tab;
+    GxTab<L, K> tab;
     tab.load(table16, threadIdx.x);
     uint32_t* back = BACK_GLOBAL ? back_ws + row * (int64_t)(T - 1) * BIG_NT : back_lds;
-    viterbi_gx<L, K, BIG_NT, DBL, BACK_GLOBAL, false, true>(x + row * ldx, T, tab, start ? start[row] : -1, buf, back,
-                                             states + row * lds, red);
+    viterbi_gx<L, K, NT, DBL, BACK_GLOBAL, false, true>(x + row * ldx, T, tab, start ? start[row] : -1, buf, back,
+                                                        states + row * lds, red);
 }
 
 template <int L, int K>
@@ -255,7 +268,7 @@ struct ViterbiRowsBig {
         constexpr bool GX = VX<L, K, BIG_NT>::R <= BIG_GX_MAX_R;
         if (T <= BIG_TV) {
             if constexpr (GX)
-                hipLaunchKernelGGL((viterbi_rows_gx_kernel<L, K, false>), dim3((unsigned)B), dim3(BIG_NT), 0, s, x, T, ldx,
+                hipLaunchKernelGGL((viterbi_rows_gx_kernel<L, K, false>), dim3((unsigned)B), dim3(gx_nt<L>()), 0, s, x, T, ldx,
                                    table16, start, states, lds, (uint32_t*)nullptr);
             else
                 hipLaunchKernelGGL((viterbi_rows_big_kernel<L, K, false>), dim3((unsigned)B), dim3(BIG_NT), 0, s, x, T, ldx,
@@ -264,7 +277,7 @@ struct ViterbiRowsBig {
             const size_t need = (size_t)B * (size_t)(T - 1) * BIG_NT * sizeof(uint32_t);
             if (!ws || ws_bytes < need) return LAMQ_EINVAL;
             if constexpr (GX)
-                hipLaunchKernelGGL((viterbi_rows_gx_kernel<L, K, true>), dim3((unsigned)B), dim3(BIG_NT), 0, s, x, T, ldx,
+                hipLaunchKernelGGL((viterbi_rows_gx_kernel<L, K, true>), dim3((unsigned)B), dim3(gx_nt<L>()), 0, s, x, T, ldx,
                                    table16, start, states, lds, (uint32_t*)ws);
             else
                 hipLaunchKernelGGL((viterbi_rows_big_kernel<L, K, true>), dim3((unsigned)B), dim3(BIG_NT), 0, s, x, T, ldx,
@@ -378,14 +391,15 @@ __global__ __launch_bounds__(BIG_NT) void ldlq_trellis_block_big_kernel(
 }
 
 // LDS of the fused minima-exchange kernel below: the block row and small arrays, the group minima (two buffers when
-// they fit, which spares each step its second barrier: 2^12 groups, and 2^13 with the back-pointers in LDS, 163,456 of
+// they fit, which spares each step its second barrier: 2^12 groups, and 2^13 with the back-pointers in LDS, 163,392 of
 // the 163,840 bytes), and the back-pointers unless they go to a workspace (BG).
 template <int L, int K, bool BG>
 constexpr int gx_lds_bytes(bool dbl)
 {
-    using V = VX<L, K, BIG_NT>;
+    constexpr int NT = gx_nt<L>();
+    using V = VX<L, K, NT>;
     return 8 * (BIG_LAZY + BIG_TV) + 8 * LAMQ_WMAX * LAMQ_WMAX + 8 * LAMQ_WMAX + 4 * BIG_TV + 4 * BIG_TV +
-           4 * 2 * (BIG_NT / 64) + 4 * (dbl ? 2 : 1) * V::R + 4 * (BG ? 1 : (BIG_TV - 1) * V::ACT);
+           4 * 2 * (NT / 64) + 4 * (dbl ? 2 : 1) * V::R + 4 * (BG ? 1 : (BIG_TV - 1) * V::step_words(32));
 }
 template <int L, int K, bool BG>
 constexpr bool gx_double_buffered() { return gx_lds_bytes<L, K, BG>(true) <= 160 * 1024; }
@@ -396,7 +410,8 @@ constexpr bool gx_double_buffered() { return gx_lds_bytes<L, K, BG>(true) <= 160
 // whose 128 KB of group minima leave no LDS for them)
 template <int L, int K, bool BG>
 struct alignas(16) GxSmem {
-    using V = VX<L, K, BIG_NT>;
+    static constexpr int NT = gx_nt<L>();
+    using V = VX<L, K, NT>;
     static constexpr bool DBL = gx_double_buffered<L, K, BG>();
     // small arrays first: their addresses stay within the 16-bit offset of LDS instructions
     double trow[BIG_LAZY + BIG_TV];
@@ -404,9 +419,9 @@ struct alignas(16) GxSmem {
     double zs[LAMQ_WMAX];
     float xs[BIG_TV];
     int path[BIG_TV];
-    float red[2 * (BIG_NT / 64)];
+    float red[2 * (NT / 64)];
     float buf[(DBL ? 2 : 1) * V::R];
-    uint32_t back[BG ? 1 : (BIG_TV - 1) * V::ACT];
+    uint32_t back[BG ? 1 : (BIG_TV - 1) * V::step_words(32)];
 };
 
 // One row's lazy block [b0, b1): `row` indexes T, S, state, states and Z; `wrow` the row's back-pointer slot in back_ws
@@ -420,7 +435,7 @@ __device__ __forceinline__ void gx_block_row(GxSmem<L, K, BG>& sm, int64_t row, 
                                              int32_t* __restrict__ states, int64_t lds, double* __restrict__ Z,
                                              int64_t ldZ, uint32_t* __restrict__ back_ws, int pre)
 {
-    using V = VX<L, K, BIG_NT>;
+    constexpr int NT = gx_nt<L>();
     constexpr bool DBL = GxSmem<L, K, BG>::DBL;
     double* trow = sm.trow;
     double* ubb = sm.ubb;
@@ -429,12 +444,12 @@ __device__ __forceinline__ void gx_block_row(GxSmem<L, K, BG>& sm, int64_t row, 
     int* path = sm.path;
     float* red = sm.red;
     float* buf = sm.buf;
-    uint32_t* back = BG ? back_ws + wrow * (int64_t)((BIG_TV - 1) * V::ACT) : sm.back;
+    uint32_t* back = BG ? back_ws + wrow * (int64_t)(BIG_BACK_WORDS) : sm.back;
     const int tid = threadIdx.x;
     const int64_t cend = (b1 + look < n) ? b1 + look : n;
-    load_block_row<BIG_NT>(trow, T + row * ldT, b0, (int)(b1 - b0), (int)(cend - b0), Z + row * ldZ - pre, pre, U,
+    load_block_row<NT>(trow, T + row * ldT, b0, (int)(b1 - b0), (int)(cend - b0), Z + row * ldZ - pre, pre, U,
                             ldU);
-    TabF16<V> tab;
+    GxTab<L, K> tab;
     tab.load(table16, tid);
     const double Sr = S[row];
     int st = state[row];
@@ -451,17 +466,18 @@ __device__ __forceinline__ void gx_block_row(GxSmem<L, K, BG>& sm, int64_t row, 
         lds_barrier();
         // the refit's U operands are fetched when the forward pass ends, under the final argmin and the traceback
         RefitRegs<4> ops;
-        const int pv = viterbi_gx<L, K, BIG_NT, DBL, BG, true>(
-            xs, TV, tab, st, buf, back, path, red, [&]() { refit_fetch_regs<BIG_NT, 4>(ops, U, ldU, j, w, nc); });
-        refit_apply_regs<BIG_NT, 4>(ops, trow, jo, w, nc, pv, table64, Sr, states + row * lds + j, Z + row * ldZ + jo, ubb,
+        const int pv = viterbi_gx<L, K, NT, DBL, BG, true>(
+            xs, TV, tab, st, buf, back, path, red, [&]() { refit_fetch_regs<NT, 4>(ops, U, ldU, j, w, nc); });
+        refit_apply_regs<NT, 4>(ops, trow, jo, w, nc, pv, table64, Sr, states + row * lds + j, Z + row * ldZ + jo, ubb,
                                zs);
         st = path[w - 1];
     }
     if (tid == 0) state[row] = st;
+    asm volatile("; k %0" ::"n"(K));  // (the widths' code in one kernel is not merged at its ends)
 }
 
 template <int L, int K, bool BG>
-__global__ __launch_bounds__(BIG_NT) void ldlq_trellis_block_gx_kernel(
+__global__ __launch_bounds__(gx_nt<L>(), gx_nt<L>() / 256) void ldlq_trellis_block_gx_kernel(
     const double* __restrict__ T, int64_t n, int64_t ldT, const double* __restrict__ U, int64_t ldU,
     const double* __restrict__ S, const double* __restrict__ table64, const uint16_t* __restrict__ table16,
     int64_t b0, int64_t b1, int width, int look, int32_t* __restrict__ state, int32_t* __restrict__ states,
@@ -519,7 +535,7 @@ __device__ __forceinline__ void gx_group_row(uint8_t* raw, const GxGroup& G, int
 }
 
 template <int L>
-__global__ __launch_bounds__(BIG_NT) void ldlq_trellis_groups_gx_kernel(
+__global__ __launch_bounds__(gx_nt<L>(), gx_nt<L>() / 256) void ldlq_trellis_groups_gx_kernel(
     const double* __restrict__ T, int64_t n, int64_t ldT, const double* __restrict__ U, int64_t ldU,
     const double* __restrict__ S, int64_t b0, int64_t b1, int width, int look, int32_t* __restrict__ state,
     int32_t* __restrict__ states, int64_t lds, double* __restrict__ Z, int64_t ldZ, int pre, GxGroups groups)
@@ -557,15 +573,15 @@ struct TrellisBlockBig {
     {
         if constexpr (VX<L, K, BIG_NT>::R <= BIG_GX_MAX_R) {
             if (gx_back_global<L, K>() && back_ws)  // the back-pointers in the workspace, two minima buffers in LDS
-                hipLaunchKernelGGL((ldlq_trellis_block_gx_kernel<L, K, true>), dim3((unsigned)m), dim3(BIG_NT), 0, s, T,
+                hipLaunchKernelGGL((ldlq_trellis_block_gx_kernel<L, K, true>), dim3((unsigned)m), dim3(gx_nt<L>()), 0, s, T,
                                    n, ldT, U, ldU, S, table64, table16, b0, b1, width, look, state, states, lds, Z, ldZ,
                                    back_ws, pre);
             else
-                hipLaunchKernelGGL((ldlq_trellis_block_gx_kernel<L, K, false>), dim3((unsigned)m), dim3(BIG_NT), 0, s, T,
+                hipLaunchKernelGGL((ldlq_trellis_block_gx_kernel<L, K, false>), dim3((unsigned)m), dim3(gx_nt<L>()), 0, s, T,
                                    n, ldT, U, ldU, S, table64, table16, b0, b1, width, look, state, states, lds, Z, ldZ,
                                    nullptr, pre);
         } else if (back_ws)
-            hipLaunchKernelGGL((ldlq_trellis_block_gx_kernel<L, K, true>), dim3((unsigned)m), dim3(BIG_NT), 0, s, T, n,
+            hipLaunchKernelGGL((ldlq_trellis_block_gx_kernel<L, K, true>), dim3((unsigned)m), dim3(gx_nt<L>()), 0, s, T, n,
                                ldT, U, ldU, S, table64, table16, b0, b1, width, look, state, states, lds, Z, ldZ, back_ws,
                                pre);
         else
@@ -628,7 +644,7 @@ static void launch_groups(const GxGroups& gg, int64_t total, double* T, int64_t 
                           int64_t ldU, const double* S, int64_t b0, int64_t b1, int width, int look, int32_t* state,
                           int32_t* states, int64_t lds, double* Z, int64_t ldZ, int pre, hipStream_t s)
 {
-    hipLaunchKernelGGL((ldlq_trellis_groups_gx_kernel<L>), dim3((unsigned)total), dim3(BIG_NT), 0, s, T, n, ldT, U, ldU,
+    hipLaunchKernelGGL((ldlq_trellis_groups_gx_kernel<L>), dim3((unsigned)total), dim3(gx_nt<L>()), 0, s, T, n, ldT, U, ldU,
                        S, b0, b1, width, look, state, states, lds, Z, ldZ, pre, gg);
 }
 
