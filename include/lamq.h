@@ -257,10 +257,13 @@ int lamq_chol_inv_upper(const double* H, int64_t n, int64_t ldH, double damp, do
 int lamq_rht_rows(const double* in, int64_t rows, int64_t n, int64_t ldi, double* out, int64_t ldo,
                   const int8_t* signs, const int8_t* A, int a, const int8_t* B, int b, int inverse, double* rms,
                   void* stream);
-int lamq_transpose_f64(const double* in, int64_t rows, int64_t cols, int64_t ldi, double* out, int64_t ldo,
-                       void* stream);
-/* Row scales S_r = max(sqrt(mean_j X[r, j]^2), 1e-12) (opgraph/codes.py:436, nested.py:168). */
-int lamq_row_rms(const double* X, int64_t rows, int64_t n, int64_t ldx, double* S, void* stream);
+
+/* The same for the factors hadamard_factors makes, known here: A the Sylvester matrix of order a = n / b, entry (i, j) =
+ * (-1)^popcount(i & j) (a B of a power-of-two order belongs to it: b = 1), and B Paley's matrix of order b. A fast
+ * Walsh-Hadamard transform takes A's place. b = 1 with n = 2^10 .. 2^13, or b = 12 or 20 with a = 16 .. 256; other shapes
+ * return LAMQ_EUNSUP (lamq_rht_rows takes them). The results differ from lamq_rht_rows's in float64 rounding only. */
+int lamq_rht_rows_sylvester(const double* in, int64_t rows, int64_t n, int64_t ldi, double* out, int64_t ldo,
+                            const int8_t* signs, int b, int inverse, double* rms, void* stream);
 
 /* ------------------------------------------------------------------------------------------------
  * Token-weighted Gram matrix on bf16 MFMA with fp32 accumulation:

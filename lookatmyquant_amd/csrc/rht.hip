@@ -497,6 +497,257 @@ extern "C" int lamq_rht_rows(const double* in, int64_t rows, int64_t n, int64_t 
     return LAMQ_OK;
 }
 
+// ------------------------------------------------------------------------------------------------ fast transforms
+// The same transform where A is the Sylvester matrix (entry (i, j) = (-1)^popcount(i & j)) of a power of two P and B is
+// small: x = M[i][j], i < P, j < b, takes the b x b products of each i and then a fast Walsh-Hadamard transform over i,
+// n (b + log2 P) additions instead of n (a + b), so that the passes over memory bound it. A thread holds 16 values in
+// registers and takes four bits of i (or fewer, its other values then independent) per stage; between stages the row
+// goes through LDS, padded so that every stage reads and writes without bank conflicts. b = 1: the row's top bits from
+// global memory as they are loaded (coalesced), then bits 0-3, then 4-7 (and, past 2^12, 8 up), whose layout stores 16
+// or more consecutive values. b = 12 and 20 (the Paley orders of widths 3 x 2^k and 5 x 2^k): a thread per i holds its
+// b values and forms the b outputs with signs known at compile time; then i's top four bits and the rest.
+// R H R^T at n = 4,096 (two of these and a transpose) 345 -> 155 us, at 2,560 238 -> 62, at 1,536 123 -> 42; larger orders
+// (b = 60, 152) stay on the matrix cores above, where the b x b products are most of the work.
+__device__ __forceinline__ double rht_scaled(double v, double s, double r)
+{
+    // v / s: the product with r = 1 / s and one correction by the exact residual (an infinity has none)
+    const double q = v * r;
+    return __builtin_isfinite(q) ? fma(fma(-q, s, v), r, q) : q;
+}
+
+// butterflies over the low W bits of u
+template <int W>
+__device__ __forceinline__ void rht_butterfly(double (&v)[16])
+{
+#pragma unroll
+    for (int w = 0; w < W; ++w)
+#pragma unroll
+        for (int u = 0; u < 16; ++u)
+            if (!(u & (1 << w))) {
+                const double a = v[u], b = v[u | (1 << w)];
+                v[u] = a + b;
+                v[u | (1 << w)] = a - b;
+            }
+}
+
+// the row's sum of squares, in a fixed order, to its RMS
+__device__ __forceinline__ void rht_row_rms(double ss, double* part, int nt, int n, double* rms)
+{
+#pragma unroll
+    for (int o = 1; o < 64; o <<= 1) ss += __shfl_xor(ss, o);
+    __syncthreads();  // (part may lie where the row was)
+    if ((threadIdx.x & 63) == 0) part[threadIdx.x >> 6] = ss;
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        double t = part[0];
+        for (int w = 1; w < nt / 64; ++w) t += part[w];
+        const double r = sqrt(t / (double)n);
+        *rms = r > 1e-12 ? r : 1e-12;
+    }
+}
+
+template <int K>
+__global__ __launch_bounds__(1 << (K - 4)) void rht_pow2_kernel(const double* in, int64_t ldi, double* out, int64_t ldo,
+                                                                const int8_t* __restrict__ signs,
+                                                                double* __restrict__ rms, double sqrt_n, int inverse)
+{
+    constexpr int N = 1 << K, NT = N / 16;
+    static_assert(K >= 10 && K <= 13, "a wave at least, 16 values a thread");
+    __shared__ double x[N + N / 16];
+    const int tid = threadIdx.x;
+    const double* xin = in + (int64_t)blockIdx.x * ldi;
+    const double rinv = 1.0 / sqrt_n;
+    const auto pad = [](int e) { return e + (e >> 4); };
+    double v[16];
+#pragma unroll
+    for (int u = 0; u < 16; ++u) v[u] = xin[tid + NT * u];
+    if (!inverse) {
+#pragma unroll
+        for (int u = 0; u < 16; ++u) v[u] = signs[tid + NT * u] > 0 ? v[u] : -v[u];
+    }
+    rht_butterfly<4>(v);  // bits K - 4 .. K - 1
+#pragma unroll
+    for (int u = 0; u < 16; ++u) x[pad(tid + NT * u)] = v[u];
+    __syncthreads();
+#pragma unroll
+    for (int u = 0; u < 16; ++u) v[u] = x[pad(16 * tid) + u];
+    rht_butterfly<4>(v);  // bits 0 .. 3
+#pragma unroll
+    for (int u = 0; u < 16; ++u) x[pad(16 * tid) + u] = v[u];
+    __syncthreads();
+    int e0 = ((tid >> 4) << 8) | (tid & 15), de = 16;  // this thread's values: e0 + de u
+#pragma unroll
+    for (int u = 0; u < 16; ++u) v[u] = x[pad(e0 + de * u)];
+    rht_butterfly<(K - 8 < 4 ? K - 8 : 4)>(v);  // bits 4 .. 7, or up to the top four
+    if constexpr (K > 12) {
+#pragma unroll
+        for (int u = 0; u < 16; ++u) x[pad(e0 + de * u)] = v[u];
+        __syncthreads();
+        e0 = ((tid >> 8) << 12) | (tid & 255);
+        de = 256;
+#pragma unroll
+        for (int u = 0; u < 16; ++u) v[u] = x[pad(e0 + de * u)];
+        rht_butterfly<(K > 12 ? K - 12 : 0)>(v);  // bits 8 up
+    }
+    double ss = 0.0;
+    double* y = out + (int64_t)blockIdx.x * ldo;
+#pragma unroll
+    for (int u = 0; u < 16; ++u) {
+        const int e = e0 + de * u;
+        double val = rht_scaled(v[u], sqrt_n, rinv);
+        if (inverse) val = signs[e] > 0 ? val : -val;
+        y[e] = val;
+        ss += val * val;
+    }
+    if (rms) rht_row_rms(ss, x, NT, N, rms + blockIdx.x);
+}
+
+// Entry (r, c) of Paley's first construction of order B = q + 1 (q prime, q = 3 mod 4): the first row +1, the first column
+// -1 below it, the rest chi((c - r) mod q) with +1 on the diagonal, chi the Legendre symbol.
+template <int B>
+constexpr bool paley_plus(int r, int c)
+{
+    if (r == 0) return true;
+    if (c == 0) return false;
+    const int q = B - 1, d = (c - r + q) % q;
+    if (d == 0) return true;
+    for (int x = 1; x < q; ++x)
+        if (x * x % q == d) return true;
+    return false;
+}
+template <int B>
+struct PaleyRows {
+    uint32_t plus[B];  // bit c of row r
+    constexpr PaleyRows() : plus()
+    {
+        for (int r = 0; r < B; ++r)
+            for (int c = 0; c < B; ++c) plus[r] |= paley_plus<B>(r, c) ? 1u << c : 0u;
+    }
+};
+
+// b = B x B products and a transform over P = 2^K values of i, 4 <= K <= 8. One row a workgroup of NT threads (whole
+// waves, at least P and n / 16 of them).
+template <int B, int K, bool inverse>
+__global__ __launch_bounds__((B * (1 << K) / 16 + 63) / 64 * 64) void rht_paley_kernel(
+    const double* in, int64_t ldi, double* out, int64_t ldo, const int8_t* __restrict__ signs, double* __restrict__ rms,
+    double sqrt_n)
+{
+    constexpr PaleyRows<B> PB;
+    constexpr int P = 1 << K, N = P * B, Q = N / 16, NT = (Q + 63) / 64 * 64, LD = B + 1;
+    static_assert(K >= 4 && K <= 8 && NT >= (P < NT ? P : NT), "the stages below");
+    __shared__ double x[P * LD];
+    __shared__ double part[NT / 64];
+    const int tid = threadIdx.x;
+    const double* xin = in + (int64_t)blockIdx.x * ldi;
+    const double rinv = 1.0 / sqrt_n;
+    for (int e0 = 0; e0 < N; e0 += 8 * NT) {
+        double v[8];
+#pragma unroll
+        for (int u = 0; u < 8; ++u) {
+            const int e = e0 + NT * u + tid;
+            v[u] = xin[e < N ? e : N - 1];
+        }
+#pragma unroll
+        for (int u = 0; u < 8; ++u) {
+            const int e = e0 + NT * u + tid;
+            if (e < N) x[e / B * LD + e % B] = (inverse || signs[e] > 0) ? v[u] : -v[u];
+        }
+    }
+    __syncthreads();
+    for (int i = tid; i < P; i += NT) {
+        double m[B];
+#pragma unroll
+        for (int j = 0; j < B; ++j) m[j] = x[i * LD + j];
+        // out[c] = sum_j B[c][j] m[j] (inverse: B[j][c])
+#pragma unroll
+        for (int c = 0; c < B; ++c) {
+            double o = 0.0;
+#pragma unroll
+            for (int j = 0; j < B; ++j) {
+                const bool plus = inverse ? (PB.plus[j] >> c) & 1u : (PB.plus[c] >> j) & 1u;
+                o = plus ? o + m[j] : o - m[j];
+            }
+            x[i * LD + c] = o;
+        }
+    }
+    __syncthreads();
+    // top four bits of i: t = r B + j, i = r + (P / 16) u
+    double v[16];
+    const int r = tid / B, j = tid - r * B;
+    if (tid < Q) {
+#pragma unroll
+        for (int u = 0; u < 16; ++u) v[u] = x[(r + (P / 16) * u) * LD + j];
+        rht_butterfly<4>(v);
+    }
+    int i0 = r, di = P / 16;
+    if constexpr (K > 4) {
+        if (tid < Q) {
+#pragma unroll
+            for (int u = 0; u < 16; ++u) x[(r + (P / 16) * u) * LD + j] = v[u];
+        }
+        __syncthreads();
+        i0 = 16 * r;
+        di = 1;
+        if (tid < Q) {
+#pragma unroll
+            for (int u = 0; u < 16; ++u) v[u] = x[(i0 + u) * LD + j];
+            rht_butterfly<(K > 4 ? K - 4 : 0)>(v);  // the low bits of i
+        }
+    }
+    double ss = 0.0;
+    if (tid < Q) {
+        double* y = out + (int64_t)blockIdx.x * ldo;
+#pragma unroll
+        for (int u = 0; u < 16; ++u) {
+            const int e = (i0 + di * u) * B + j;
+            double val = rht_scaled(v[u], sqrt_n, rinv);
+            if (inverse) val = signs[e] > 0 ? val : -val;
+            y[e] = val;
+            ss += val * val;
+        }
+    }
+    if (rms) rht_row_rms(ss, part, NT, N, rms + blockIdx.x);
+}
+
+extern "C" int lamq_rht_rows_sylvester(const double* in, int64_t rows, int64_t n, int64_t ldi, double* out, int64_t ldo,
+                                       const int8_t* signs, int b, int inverse, double* rms, void* stream)
+{
+    if (!in || !out || !signs || rows < 0 || n < 1 || ldi < n || ldo < n || b < 1 || n % b) return LAMQ_EINVAL;
+    const int64_t P = n / b;
+    if (P & (P - 1)) return LAMQ_EINVAL;
+    if (rows > 0x7fffffff) return LAMQ_EUNSUP;
+    int k = 0;
+    while (((int64_t)1 << k) < P) ++k;
+    const bool ok = b == 1 ? (k >= 10 && k <= 13) : ((b == 12 || b == 20) && k >= 4 && k <= 8);
+    if (!ok) return LAMQ_EUNSUP;
+    if (rows == 0) return LAMQ_OK;
+    const dim3 grid((unsigned)rows);
+    hipStream_t s = as_stream(stream);
+    const double sqrt_n = sqrt((double)n);
+#define RHT_POW2(KK)                                                                                                   \
+    if (b == 1 && k == KK)                                                                                             \
+        hipLaunchKernelGGL(rht_pow2_kernel<KK>, grid, dim3(1 << (KK - 4)), 0, s, in, ldi, out, ldo, signs, rms, sqrt_n, \
+                           inverse);
+#define RHT_PALEY1(BB, KK, INV)                                                                                        \
+    hipLaunchKernelGGL((rht_paley_kernel<BB, KK, INV>), grid, dim3((BB * (1 << KK) / 16 + 63) / 64 * 64), 0, s, in, ldi, \
+                       out, ldo, signs, rms, sqrt_n)
+#define RHT_PALEY(BB, KK)                                                                                              \
+    if (b == BB && k == KK) {                                                                                          \
+        if (inverse)                                                                                                   \
+            RHT_PALEY1(BB, KK, true);                                                                                  \
+        else                                                                                                           \
+            RHT_PALEY1(BB, KK, false);                                                                                 \
+    }
+    RHT_POW2(10) RHT_POW2(11) RHT_POW2(12) RHT_POW2(13)
+    RHT_PALEY(12, 4) RHT_PALEY(12, 5) RHT_PALEY(12, 6) RHT_PALEY(12, 7) RHT_PALEY(12, 8)
+    RHT_PALEY(20, 4) RHT_PALEY(20, 5) RHT_PALEY(20, 6) RHT_PALEY(20, 7) RHT_PALEY(20, 8)
+#undef RHT_POW2
+#undef RHT_PALEY
+#undef RHT_PALEY1
+    LAMQ_LAUNCH_CHECK();
+    return LAMQ_OK;
+}
+
 __global__ __launch_bounds__(256) void transpose_f64_kernel(const double* __restrict__ in, int64_t rows, int64_t cols,
                                                             int64_t ldi, double* __restrict__ out, int64_t ldo)
 {

@@ -119,13 +119,29 @@ def rht_rows(X: torch.Tensor, seed: int, inverse: bool = False, want_rms: bool =
     need(X, torch.float64, "X", 2)
     rows, n = X.shape
     dev = str(X.device)
-    A, B = _factors(n, dev)
     s = _signs(n, seed, dev)
     y = torch.empty_like(X, memory_format=torch.contiguous_format) if out is None else out
     rms = torch.empty(rows, dtype=torch.float64, device=X.device) if want_rms else None
+    b = fast_factor(n)
+    if b:
+        check(lib().lamq_rht_rows_sylvester(ptr(X), rows, n, ld(X), ptr(y), ld(y), ptr(s), b, 1 if inverse else 0, ptr(rms),
+                                            stream(X.device)), "rht_rows")
+        return (y, rms) if want_rms else y
+    A, B = _factors(n, dev)
     check(lib().lamq_rht_rows(ptr(X), rows, n, ld(X), ptr(y), ld(y), ptr(s), ptr(A), A.shape[0], ptr(B), B.shape[0],
                               1 if inverse else 0, ptr(rms), stream(X.device)), "rht_rows")
     return (y, rms) if want_rms else y
+
+
+@lru_cache(maxsize=64)
+def fast_factor(n: int) -> int:
+    """The order b of the factor that lamq_rht_rows_sylvester multiplies out, its transform taking the rest of n (0: n
+    goes to lamq_rht_rows). hadamard_factors' A is always a Sylvester matrix; so is a B whose order is a power of two,
+    and the two together are one of order n (b = 1); any other B is Paley's."""
+    a, b = _factor_sizes(n)
+    if b & (b - 1) == 0:
+        return 1 if 1 << 10 <= n <= 1 << 13 else 0
+    return b if b in (12, 20) and 16 <= a <= 256 else 0
 
 
 def device_rows(groups: list, dev) -> list:

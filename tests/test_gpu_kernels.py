@@ -418,6 +418,30 @@ def test_rht_rows(E, m, n, seed):
     assert np.abs(back - W).max() < 1e-12 * np.abs(W).max()
 
 
+@pytest.mark.parametrize("n", [1024, 2048, 4096, 8192, 192, 384, 768, 1536, 3072, 320, 640, 1280, 2560, 5120])
+def test_rht_rows_fast_transform_matches_products(E, monkeypatch, n):
+    """Every width the fast transform takes, forward and inverse, row scales, strided rows and in place, against the
+    general path's products. Bound: each path sums at most a + b (or log2) terms of magnitude up to sum |x| / sqrt(n)
+    per output, so they differ by at most 2 (a + b + 4) 2^-53 of it."""
+    rng = np.random.default_rng(n)
+    a, b = E._factor_sizes(n)
+    assert E.fast_factor(n) == (1 if b & (b - 1) == 0 else b)
+    W = cuda(rng.standard_normal((5, n + 6)) * 10.0 ** rng.integers(-3, 4, (5, 1)))[:, :n]
+    out = torch.full((5, n + 2), 7.0, dtype=torch.float64, device="cuda")
+    say(f"rht rows {n}")
+    got, rms = E.rht_rows(W, 3, want_rms=True)
+    E.rht_rows(W, 3, inverse=True, out=out[:, :n])
+    here = W.contiguous()
+    E.rht_rows(here, 3, out=here)
+    monkeypatch.setattr(E, "fast_factor", lambda n: 0)
+    want, wrms = E.rht_rows(W, 3, want_rms=True)
+    back = E.rht_rows(W, 3, inverse=True)
+    tol = 2 * (a + b + 4) * 2.0 ** -53 * W.abs().sum(1, keepdim=True) / n ** 0.5
+    assert bool(((got - want).abs() <= tol).all()) and bool(((out[:, :n] - back).abs() <= tol).all())
+    assert torch.equal(here, got) and bool((out[:, n:] == 7.0).all())
+    assert bool(((rms - wrms).abs() <= tol[:, 0]).all())
+
+
 def test_rotate_hessian(E, config12):
     _, H = config12
     say("rotate hessian n=960")
