@@ -4,12 +4,21 @@
 // the key blocks of 64 up to its last query: each block's K and V rows (16 KB each) go straight from memory into LDS
 // (global_load_lds, 16 bytes a lane, no registers), double-buffered, the next block's loads issued as soon as the
 // current one is published (one barrier a block), so the four waves share one copy and no wave waits on a global
-// load. Per 32-key half of a block a wave forms S^T = K Q^T (32 keys x 32 queries: the head dim, 128, as eight
-// 16-deep steps of v_mfma_f32_32x32x16_bf16, float32 sums), masks it causally, updates each query's running maximum
-// and sum (the online softmax: exp2 with the scale and log2(e) folded into the scores), rounds the probabilities to
-// bf16 and accumulates O^T += V^T P^T (128 x 32, float32) with the earlier sums rescaled; a wave past its own last
-// query skips the half (its key blocks still arrive for the others). At the end O = O^T / sum, rounded to bf16
+// load. Per block a wave forms S^T = K Q^T (two tiles of 32 keys x 32 queries: the head dim, 128, as eight 16-deep steps of
+// v_mfma_f32_32x32x16_bf16 each, float32 sums), masks it where the block reaches past its first query, updates each
+// query's maximum and its lanes' parts of the sum (the online softmax: exp2 with the scale and log2(e) folded into one
+// multiply-add a score), rounds the probabilities to bf16 and accumulates O^T += V^T P^T (128 x 32, float32); a wave past
+// its own last query skips the block (which still arrives for the others). At the end O = O^T / sum, rounded to bf16
 // (nearest, ties to even).
+//
+// What bounds it: with two waves a SIMD the vector work of one runs under the matrix work of the other, 1,024 clocks a
+// block, so the vector chain of a block is kept short: 64 keys a softmax instead of 32, no mask off the diagonal, the
+// earlier sums rescaled only when some query's maximum has grown (a lag of 2^8 allowed would save 5%, but the largest
+// probability is then no longer exactly 1 before its rounding to bf16), the halves of a query's keys combined by a swap of the wave's halves (LDS shuffles
+// before) and its sum only at the end, row pointers advanced a block at a time, and V's transposing reads issued before
+// the softmax they are needed after. 8 x 32 heads x 2,048: 655 -> 330 us (833 TFLOP/s); 32 sequences 2.56 -> 1.29 ms.
+// Workgroups go out pair by pair of sequence and key/value head, pairs spread over the XCDs, so that the query heads and
+// blocks that read the same K and V run on one XCD together.
 //
 // Operand layouts (32x32x16 bf16 MFMA): A[m][k] has lane l holding m = l % 32 and k = 8 (l / 32) .. + 7; B[k][n]
 // has lane l holding n = l % 32 and the same k; the result has lane l holding column l % 32 and rows
@@ -44,40 +53,86 @@ __device__ __forceinline__ uint32_t at_ksw(int row, int chunk)
     return (uint32_t)(row * (AT_D * 2) + ((chunk ^ (row & 15)) << 4));
 }
 
+typedef short lamq_at_s4 __attribute__((ext_vector_type(4)));
+typedef __attribute__((address_space(3))) lamq_at_s4 lamq_at_lds_s4;
+
+// the larger of this lane's value and lane ^ 32's (one swap of the wave's halves, no LDS)
+__device__ __forceinline__ float at_max32(float v)
+{
+    const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+    return fmaxf(__uint_as_float(r[0]), __uint_as_float(r[1]));
+}
+__device__ __forceinline__ float at_sum32(float v)
+{
+    const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+    return __uint_as_float(r[0]) + __uint_as_float(r[1]);
+}
+
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) void attention_causal_kernel(
     const uint16_t* __restrict__ Q, int64_t sqb, int64_t sqh, int64_t sqt, const uint16_t* __restrict__ K,
     int64_t skb, int64_t skh, int64_t skt, const uint16_t* __restrict__ V, int64_t svb, int64_t svh, int64_t svt,
-    uint16_t* __restrict__ O, int64_t sob, int64_t soh, int64_t sot, int rep, int T, float scale_log2)
+    uint16_t* __restrict__ O, int64_t sob, int64_t soh, int64_t sot, int rep, int Hkv, int pairs, int T, float scale_log2)
 {
     __shared__ __align__(16) uint8_t lds[2][2][AT_OPB];  // [buffer][K, V]
     const int nqb = (T + AT_QB - 1) / AT_QB;
-    const int qb = nqb - 1 - (int)blockIdx.x;  // the longest query blocks first
-    const int h = (int)blockIdx.y, b = (int)blockIdx.z;
+    // workgroup -> (pair of sequence and key/value head, query head of the pair, query block)
+    int pair, rem;
+    {
+        const int id = (int)blockIdx.x, per = nqb * rep;
+        if (pairs % LAMQ_XCDS == 0) {
+            const int y = id / LAMQ_XCDS;
+            pair = y / per * LAMQ_XCDS + id % LAMQ_XCDS;
+            rem = y % per;
+        } else {
+            pair = id / per;
+            rem = id % per;
+        }
+    }
+    const int qb = nqb - 1 - rem / rep;  // the longest query blocks first
+    const int b = pair / Hkv, hk = pair % Hkv, h = hk * rep + rem % rep;
     const int wave = (int)(threadIdx.x >> 6), lane = (int)(threadIdx.x & 63);
     const int wv = __builtin_amdgcn_readfirstlane(wave);
-    const int q0 = qb * AT_QB + AT_QW * wave;
+    const int q0 = qb * AT_QB + AT_QW * wv;
     const int li = lane & 31, hi = lane >> 5, g = lane >> 4, i16 = lane & 15;
     const uint16_t* Qp = Q + b * sqb + (int64_t)h * sqh;
-    const uint16_t* Kp = K + b * skb + (int64_t)(h / rep) * skh;
-    const uint16_t* Vp = V + b * svb + (int64_t)(h / rep) * svh;
+    const uint16_t* Kp = K + b * skb + (int64_t)hk * skh;
+    const uint16_t* Vp = V + b * svb + (int64_t)hk * svh;
     const uint32_t base = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) uint8_t*)lds;
     // every wave takes part in the loads and barriers up to the workgroup's last query; a wave's own work ends at its
     // last query (none for a wave wholly past T)
     const int wg_last = (qb * AT_QB + AT_QB < T ? qb * AT_QB + AT_QB : T) - 1;
     const int nblk = wg_last / AT_KB2 + 1;
     const int my_last = q0 < T ? (q0 + AT_QW < T ? q0 + AT_QW : T) - 1 : -1;
-    // block kb's rows (keys past T read row T - 1: finite values that meet zero probabilities) into buffer kb & 1:
-    // instruction i (four a wave and operand) covers rows 4i .. 4i + 3, lane l row 4i + l / 16, slot l % 16
+    // block kb's rows into buffer kb & 1: instruction i (four a wave and operand) covers rows 4i .. 4i + 3, lane l row
+    // 4i + l / 16, slot l % 16. The row pointers advance a block at a time; in a block that reaches past T the rows there
+    // read row T - 1 (finite values that meet zero probabilities)
+    const int lrow = 16 * wv + (lane >> 4), slot = lane & 15;
+    const uint16_t* kp[4];
+    const uint16_t* vp[4];
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+        const int row = lrow + 4 * q;
+        kp[q] = Kp + row * skt + 8 * (slot ^ (row & 15));
+        vp[q] = Vp + row * svt + 8 * (slot ^ (4 * (row & 3)));
+    }
     auto load_block = [&](int kb) {
-        const int k0 = kb * AT_KB2;
         const uint32_t kbuf = base + (uint32_t)((kb & 1) * 2 * AT_OPB), vbuf = kbuf + AT_OPB;
+        const int over = kb * AT_KB2 + AT_KB2 - T;  // rows past T
 #pragma unroll
         for (int q = 0; q < 4; ++q) {
             const int i = 4 * wv + q;
-            const int row = 4 * i + (lane >> 4), slot = lane & 15;
-            const int64_t key = k0 + row < T ? k0 + row : T - 1;
-            load_lds16(Kp + key * skt + 8 * (slot ^ (row & 15)), kbuf + (uint32_t)(i * 1024));
-            load_lds16(Vp + key * svt + 8 * (slot ^ (4 * (row & 3))), vbuf + (uint32_t)(i * 1024));
+            const uint16_t *ka = kp[q], *va = vp[q];
+            if (over > 0) {  // uniform
+                const int back = lrow + 4 * q - (AT_KB2 - 1 - over);  // this row's distance past row T - 1
+                if (back > 0) {
+                    ka -= back * skt;
+                    va -= back * svt;
+                }
+            }
+            load_lds16(ka, kbuf + (uint32_t)(i * 1024));
+            load_lds16(va, vbuf + (uint32_t)(i * 1024));
+            kp[q] += AT_KB2 * skt;
+            vp[q] += AT_KB2 * svt;
         }
     };
     load_block(0);
@@ -96,58 +151,35 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
     for (int t = 0; t < 4; ++t)
 #pragma unroll
         for (int v = 0; v < 16; ++v) o[t][v] = 0.0f;
-    float mrun = -__builtin_inff(), lrun = 0.0f;
-    using v2u = uint32_t __attribute__((ext_vector_type(2)));
+    float mrun = -__builtin_inff(), lrun = 0.0f;  // the maximum (of the scaled scores), this lane's part of the sum
     for (int kb = 0; kb < nblk; ++kb) {
         wait_vm<0>();     // this wave's loads of block kb have landed
         __syncthreads();  // everyone's; the other buffer (block kb - 1) is free
         if (kb + 1 < nblk) load_block(kb + 1);
+        const int k0 = kb * AT_KB2;
+        if (k0 > my_last) continue;  // uniform: this wave's queries end before these keys
         const uint8_t* kl = lds[kb & 1][0];
         const uint32_t vbase = base + (uint32_t)(((kb & 1) * 2 + 1) * AT_OPB);
-        for (int hf = 0; hf < 2; ++hf) {
-            const int k0 = kb * AT_KB2 + AT_KB * hf;
-            if (k0 > my_last) break;  // uniform: this wave's queries end before these keys
-            // K fragments (A of S^T): key 32 hf + li of the block, head dims 16 j + 8 hi .. + 7 (chunk 2 j + hi)
-            lamq_at_bf16x8 kf[8];
+        // S^T, two tiles of 32 keys: K fragments (A) of key 32 hf + li, head dims 16 j + 8 hi .. + 7 (chunk 2 j + hi)
+        lamq_at_f32x16 s[2];
 #pragma unroll
-            for (int j = 0; j < 8; ++j)
-                kf[j] = *reinterpret_cast<const lamq_at_bf16x8*>(kl + at_ksw(AT_KB * hf + li, 2 * j + hi));
-            lamq_at_f32x16 s;
+        for (int hf = 0; hf < 2; ++hf)
 #pragma unroll
-            for (int v = 0; v < 16; ++v) s[v] = 0.0f;
+            for (int v = 0; v < 16; ++v) s[hf][v] = 0.0f;
 #pragma unroll
-            for (int j = 0; j < 8; ++j) s = __builtin_amdgcn_mfma_f32_32x32x16_bf16(kf[j], qf[j], s, 0, 0, 0);
-            // causal mask, scale, the running maximum of each query (its 32 keys: 16 here, 16 in lane l ^ 32)
-            float mx = -__builtin_inff();
+        for (int j = 0; j < 8; ++j)
 #pragma unroll
-            for (int v = 0; v < 16; ++v) {
-                const int key = k0 + 8 * (v >> 2) + 4 * hi + (v & 3);
-                const float x = (key <= myq && key < T) ? s[v] * scale_log2 : -__builtin_inff();
-                s[v] = x;
-                mx = fmaxf(mx, x);
+            for (int hf = 0; hf < 2; ++hf) {
+                const lamq_at_bf16x8 kf =
+                    *reinterpret_cast<const lamq_at_bf16x8*>(kl + at_ksw(AT_KB * hf + li, 2 * j + hi));
+                s[hf] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(kf, qf[j], s[hf], 0, 0, 0);
             }
-            mx = fmaxf(mx, __shfl_xor(mx, 32));
-            const float mnew = fmaxf(mrun, mx);  // finite from the first half on: key 0 is never masked
-            const float alpha = __builtin_amdgcn_exp2f(mrun - mnew);  // 0 on the first half
-            float ps = 0.0f;
-            lamq_at_bf16x8 pf[2];
+        // V fragments, sixteen transposing reads a half, under the softmax. Lane: head dim 32 t + li; keys 16 mi + 4 hi +
+        // {0..3} and + 8 of the half (the P^T order); the group's lane i16 points at row 32 hf + 16 mi + 4 hi + i16 / 4,
+        // columns 32 t + 16 (g & 1) + 4 (i16 % 4) .. + 3
+        lamq_at_s4 vf[2][4][2][2];
 #pragma unroll
-            for (int v = 0; v < 16; ++v) {
-                const float p = __builtin_amdgcn_exp2f(s[v] - mnew);  // masked: exp2(-inf) = 0
-                ps += p;
-                pf[v >> 3][v & 7] = (__bf16)p;
-            }
-            ps += __shfl_xor(ps, 32);
-            lrun = lrun * alpha + ps;
-            mrun = mnew;
-#pragma unroll
-            for (int t = 0; t < 4; ++t)
-#pragma unroll
-                for (int v = 0; v < 16; ++v) o[t][v] *= alpha;
-            // all sixteen transposing reads first, one wait, then the eight MFMAs. Lane: head dim 32 t + li; keys
-            // 16 mi + 4 hi + {0..3} and + 8 of the half (the P^T order); the group's lane i16 points at row
-            // 32 hf + 16 mi + 4 hi + i16 / 4, columns 32 t + 16 (g & 1) + 4 (i16 % 4) .. + 3
-            v2u lo[4][2], hi2[4][2];
+        for (int hf = 0; hf < 2; ++hf)
 #pragma unroll
             for (int t = 0; t < 4; ++t)
 #pragma unroll
@@ -156,34 +188,61 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
                     const int col = 32 * t + 16 * (g & 1) + 4 * (i16 & 3);
                     const uint32_t a0 = vbase + at_sw(row, col >> 3) + 8 * ((col >> 2) & 1);
                     const uint32_t a1 = vbase + at_sw(row + 8, col >> 3) + 8 * ((col >> 2) & 1);
-                    // early-clobber outputs: the first read's destination may not share the second's address
-                    // register (the first can return into it before the second read leaves the wave)
-                    asm volatile("ds_read_b64_tr_b16 %0, %2\n\tds_read_b64_tr_b16 %1, %3"
-                                 : "=&v"(lo[t][mi]), "=&v"(hi2[t][mi])
-                                 : "v"(a0), "v"(a1)
-                                 : "memory");
+                    vf[hf][t][mi][0] = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lamq_at_lds_s4*)(uintptr_t)a0);
+                    vf[hf][t][mi][1] = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lamq_at_lds_s4*)(uintptr_t)a1);
                 }
-            asm volatile("s_waitcnt lgkmcnt(0)"
-                         : "+v"(lo[0][0]), "+v"(lo[0][1]), "+v"(lo[1][0]), "+v"(lo[1][1]), "+v"(lo[2][0]),
-                           "+v"(lo[2][1]), "+v"(lo[3][0]), "+v"(lo[3][1]), "+v"(hi2[0][0]), "+v"(hi2[0][1]),
-                           "+v"(hi2[1][0]), "+v"(hi2[1][1]), "+v"(hi2[2][0]), "+v"(hi2[2][1]), "+v"(hi2[3][0]),
-                           "+v"(hi2[3][1])
-                         :
-                         : "memory");
+        // the causal mask, only where the block reaches past the wave's first query (a key past T is past every query
+        // below T too)
+        if (k0 + AT_KB2 - 1 > q0) {
+#pragma unroll
+            for (int hf = 0; hf < 2; ++hf)
+#pragma unroll
+                for (int v = 0; v < 16; ++v) {
+                    const int key = k0 + AT_KB * hf + 8 * (v >> 2) + 4 * hi + (v & 3);
+                    s[hf][v] = key <= myq ? s[hf][v] : -__builtin_inff();
+                }
+        }
+        float mx = fmaxf(s[0][0], s[1][0]);
+#pragma unroll
+        for (int v = 1; v < 16; ++v) mx = fmaxf(fmaxf(mx, s[0][v]), s[1][v]);
+        const float ms = at_max32(mx) * scale_log2;
+        // the sums are rescaled only in blocks where some query's maximum grows
+        if (__builtin_amdgcn_ballot_w64(ms > mrun)) {
+            const float mnew = fmaxf(mrun, ms);  // finite from the first block on: key 0 is never masked
+            const float alpha = __builtin_amdgcn_exp2f(mrun - mnew);  // 0 on the first block
+            lrun *= alpha;
+            mrun = mnew;
 #pragma unroll
             for (int t = 0; t < 4; ++t)
 #pragma unroll
-                for (int mi = 0; mi < 2; ++mi) {
-                    const uint32_t __attribute__((ext_vector_type(4))) w = {lo[t][mi][0], lo[t][mi][1], hi2[t][mi][0],
-                                                                            hi2[t][mi][1]};
-                    o[t] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(lamq_at_bf16x8, w), pf[mi], o[t], 0,
-                                                                   0, 0);
-                }
+                for (int v = 0; v < 16; ++v) o[t][v] *= alpha;
         }
+        lamq_at_bf16x8 pf[2][2];
+        float ps[4] = {0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+        for (int hf = 0; hf < 2; ++hf)
+#pragma unroll
+            for (int v = 0; v < 16; ++v) {
+                const float p = __builtin_amdgcn_exp2f(fmaf(s[hf][v], scale_log2, -mrun));  // masked: exp2(-inf) = 0
+                ps[v & 3] += p;
+                pf[hf][v >> 3][v & 7] = (__bf16)p;
+            }
+        lrun += (ps[0] + ps[1]) + (ps[2] + ps[3]);
+#pragma unroll
+        for (int hf = 0; hf < 2; ++hf)
+#pragma unroll
+            for (int mi = 0; mi < 2; ++mi)
+#pragma unroll
+                for (int t = 0; t < 4; ++t) {
+                    const short __attribute__((ext_vector_type(8))) w =
+                        __builtin_shufflevector(vf[hf][t][mi][0], vf[hf][t][mi][1], 0, 1, 2, 3, 4, 5, 6, 7);
+                    o[t] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(lamq_at_bf16x8, w), pf[hf][mi], o[t],
+                                                                   0, 0, 0);
+                }
         // the next iteration's barrier comes after every wave's reads of this buffer (their results are used above)
     }
     if (myq >= T) return;
-    const float inv = 1.0f / lrun;
+    const float inv = 1.0f / at_sum32(lrun);
     uint16_t* Op = O + b * sob + (int64_t)h * soh + (int64_t)myq * sot;
 #pragma unroll
     for (int t = 0; t < 4; ++t)
@@ -217,9 +276,10 @@ extern "C" int lamq_attention_causal_bf16(const uint16_t* q, int64_t sqb, int64_
     if (((uintptr_t)q % 16) || ((uintptr_t)k % 16) || ((uintptr_t)v % 16) || ((uintptr_t)out % 8)) return LAMQ_EINVAL;
     if (B == 0 || T == 0) return LAMQ_OK;
     if (B > 65535 || H > 65535 || T > 0x7fffff) return LAMQ_EUNSUP;
-    const dim3 grid((unsigned)cdiv(T, AT_QB), (unsigned)H, (unsigned)B);
+    if (cdiv(T, AT_QB) * H * B > 0x7fffffff) return LAMQ_EUNSUP;
+    const dim3 grid((unsigned)(cdiv(T, AT_QB) * H * B));
     hipLaunchKernelGGL(attention_causal_kernel, grid, dim3(256), 0, as_stream(stream), q, sqb, sqh, sqt, k, skb, skh, skt,
-                       v, svb, svh, svt, out, sob, soh, sot, (int)(H / Hkv), (int)T, scale * 1.4426950408889634f);
+                       v, svb, svh, svt, out, sob, soh, sot, (int)(H / Hkv), (int)Hkv, (int)(B * Hkv), (int)T, scale * 1.4426950408889634f);
     LAMQ_LAUNCH_CHECK();
     return LAMQ_OK;
 }

@@ -172,6 +172,26 @@ def test_rms_norm_matches_the_float32_chain(shape):
     assert (got == ref).float().mean().item() > 0.99
 
 
+@pytest.mark.parametrize("B,H,Hkv,T,trend", [(1, 3, 1, 130, 40.0), (2, 8, 4, 65, -40.0), (3, 2, 2, 63, 40.0),
+                                              (1, 1, 1, 257, 300.0), (4, 4, 2, 200, 0.0)])
+def test_fused_attention_growing_scores_and_edges(B, H, Hkv, T, trend):
+    """Scores that rise or fall along the keys (the running maximum grows in every block, or never after the first),
+    block edges, and pair counts that are and are not a multiple of the XCDs, against float64. Bound: the probabilities
+    and the result are rounded to bf16 (2^-9 of each), so an output is within 2^-8 sum p |v| up to float32 sums: 2^-7."""
+    from lookatmyquant_amd import engine as E
+
+    g = torch.Generator(device="cuda").manual_seed(T)
+    q, k, v = (torch.randn(B, h, T, 128, generator=g, device="cuda") for h in (H, Hkv, Hkv))
+    q[..., 0] = 8.0
+    k[..., 0] = trend * torch.arange(T, device="cuda") / T
+    q, k, v = (t.to(torch.bfloat16) for t in (q, k, v))
+    got = E.attention_causal(q, k, v, 128 ** -0.5).double().cpu()
+    kk, vv = (t.double().cpu().repeat_interleave(H // Hkv, 1) for t in (k, v))
+    P = q.double().cpu() @ kk.transpose(-1, -2).contiguous() * 128 ** -0.5
+    P = P.masked_fill(torch.ones(T, T, dtype=torch.bool).triu(1), -torch.inf).softmax(-1)
+    assert bool(((got - P @ vv).abs() <= 2.0 ** -7 * (P @ vv.abs())).all())
+
+
 @pytest.mark.parametrize("B,H,Hkv,T", [(2, 32, 8, 2048), (3, 4, 4, 33), (1, 8, 2, 1)])
 def test_fused_attention_shapes_against_float64(B, H, Hkv, T):
     """The fused attention at the config-5 shape (GQA 32/8, T = 2,048), a ragged T with one query block partly past it
