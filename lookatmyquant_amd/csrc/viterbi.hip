@@ -2,7 +2,7 @@
 // block-LDLQ sweep (the search fused with the block's fp64 refit).
 #include "trellis.h"
 
-#define LAMQ_TV_LDS 32  // longest standalone path whose back-pointers stay in LDS
+#define LAMQ_TV_LDS 32  // longest standalone path that needs no workspace
 #define LAMQ_TV_BLK 24  // longest search of the fused block (width + look)
 #define LAMQ_LAZY_MAX 128
 // Workgroups of the fused block a CU holds (four waves each, one per SIMD). A row's search alternates steps that fill
@@ -15,7 +15,14 @@
 // ------------------------------------------------------------------------------------------------
 // viterbi_rows: one workgroup per row (opgraph/codes.py:151-181).
 // ------------------------------------------------------------------------------------------------
-template <int L, int K, bool BACK_GLOBAL>
+// A path's targets are staged in LDS (up to LAMQ_TV_STAGE; beyond, they are read from memory as the steps need them, each
+// read then waiting for the back-pointer stores before it as well). Its back-pointers lie in LDS where they fit and the
+// rows all fit on the chip so (a byte per group owner and step: 64 KB at 256 positions of L = 12), else in the workspace:
+// the steps do not wait for them there, but the traceback takes a round trip to memory per three positions instead of
+// one to LDS. 256 paths of 256 positions at L = 12 (one a CU), k = 1 .. 4: 109, 99, 114 and 122 us with both in memory,
+// 110, 99, 106 and 117 with the targets staged, 96, 92, 89 and 104 with the back-pointers in LDS too.
+#define LAMQ_TV_STAGE 1024
+template <int L, int K, bool BACK_GLOBAL, bool STAGE>
 __global__ __launch_bounds__(LAMQ_NT) void viterbi_rows_kernel(const float* __restrict__ x, int T, int64_t ldx,
                                                                const float* __restrict__ C,
                                                                const int32_t* __restrict__ start,
@@ -23,16 +30,28 @@ __global__ __launch_bounds__(LAMQ_NT) void viterbi_rows_kernel(const float* __re
                                                                uint8_t* __restrict__ back_ws)
 {
     using V = VX<L, K, LAMQ_NT>;
+    extern __shared__ __align__(16) float dyn[];  // STAGE: T targets (to 16 bytes); then the back-pointers in LDS
     __shared__ __align__(16) float buf[2 * V::R];
-    __shared__ uint8_t back_lds[BACK_GLOBAL ? 1 : (LAMQ_TV_LDS - 1) * V::ACT];
     __shared__ __align__(8) float red[2 * (LAMQ_NT / 64)];
     const int64_t row = blockIdx.x;
     const int tid = threadIdx.x;
     TabF32<V> tab;
     if (tid < V::ACT) tab.load(C, tid);
-    uint8_t* back = BACK_GLOBAL ? back_ws + row * (int64_t)(T - 1) * V::ACT : back_lds;
+    const float* xr = x + row * ldx;
     const int st = start ? start[row] : -1;
-    viterbi_gx<L, K, LAMQ_NT, true, BACK_GLOBAL, false, true>(x + row * ldx, T, tab, st, buf, back, states + row * lds, red);
+    if constexpr (STAGE) {
+        for (int t = tid; t < T; t += LAMQ_NT) dyn[t] = search_target(xr[t]);
+        __syncthreads();
+        if constexpr (BACK_GLOBAL)
+            viterbi_gx<L, K, LAMQ_NT, true, true>(dyn, T, tab, st, buf, back_ws + row * (int64_t)(T - 1) * V::ACT,
+                                                  states + row * lds, red);
+        else
+            viterbi_gx<L, K, LAMQ_NT, true, false>(dyn, T, tab, st, buf, reinterpret_cast<uint8_t*>(dyn + (T + 3) / 4 * 4),
+                                                   states + row * lds, red);
+    } else {
+        viterbi_gx<L, K, LAMQ_NT, true, true, false, true>(xr, T, tab, st, buf, back_ws + row * (int64_t)(T - 1) * V::ACT,
+                                                           states + row * lds, red);
+    }
 }
 
 template <int L, int K>
@@ -40,13 +59,25 @@ struct ViterbiRows {
     static int run(const float* x, int64_t B, int T, int64_t ldx, const float* C, const int32_t* start,
                    int32_t* states, int64_t lds, void* ws, size_t ws_bytes, hipStream_t s)
     {
-        if (T <= LAMQ_TV_LDS) {
-            hipLaunchKernelGGL((viterbi_rows_kernel<L, K, false>), dim3((unsigned)B), dim3(LAMQ_NT), 0, s, x, T, ldx, C,
-                               start, states, lds, (uint8_t*)nullptr);
+        using V = VX<L, K, LAMQ_NT>;
+        constexpr size_t CU_LDS = 160 * 1024, FIXED = 4 * 2 * V::R + 4 * 2 * (LAMQ_NT / 64);
+        constexpr int64_t CUS = 256;
+        const size_t need = T <= LAMQ_TV_LDS ? 0 : (size_t)B * (size_t)T * V::ACT;
+        if (need && (!ws || ws_bytes < need)) return LAMQ_EINVAL;
+        const size_t xb = 16 * ((size_t)(T + 3) / 4), bb = (size_t)(T - 1) * V::ACT;
+        const bool fits = FIXED + xb + bb <= CU_LDS;
+        if (T <= LAMQ_TV_LDS ||
+            (T <= LAMQ_TV_STAGE && fits && B <= CUS * (int64_t)(CU_LDS / (FIXED + xb + bb)))) {
+            if (FIXED + xb + bb > 48 * 1024)
+                LAMQ_HIP_CHECK(hipFuncSetAttribute((const void*)viterbi_rows_kernel<L, K, false, true>,
+                                                   hipFuncAttributeMaxDynamicSharedMemorySize, (int)(CU_LDS - FIXED)));
+            hipLaunchKernelGGL((viterbi_rows_kernel<L, K, false, true>), dim3((unsigned)B), dim3(LAMQ_NT), xb + bb, s, x, T,
+                               ldx, C, start, states, lds, (uint8_t*)nullptr);
+        } else if (T <= LAMQ_TV_STAGE) {
+            hipLaunchKernelGGL((viterbi_rows_kernel<L, K, true, true>), dim3((unsigned)B), dim3(LAMQ_NT), xb, s, x, T, ldx, C,
+                               start, states, lds, (uint8_t*)ws);
         } else {
-            const size_t need = (size_t)B * (size_t)T * VX<L, K, LAMQ_NT>::ACT;
-            if (!ws || ws_bytes < need) return LAMQ_EINVAL;
-            hipLaunchKernelGGL((viterbi_rows_kernel<L, K, true>), dim3((unsigned)B), dim3(LAMQ_NT), 0, s, x, T, ldx, C,
+            hipLaunchKernelGGL((viterbi_rows_kernel<L, K, true, false>), dim3((unsigned)B), dim3(LAMQ_NT), 0, s, x, T, ldx, C,
                                start, states, lds, (uint8_t*)ws);
         }
         LAMQ_LAUNCH_CHECK();

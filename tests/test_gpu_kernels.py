@@ -137,6 +137,25 @@ def test_viterbi_nan_and_infinite_targets_match_oracle(E, L, k):
     assert np.array_equal(got, O.viterbi(x, tab, L, k, start=st))
 
 
+@pytest.mark.parametrize("L,k,B,T", [(12, 2, 3, 33), (12, 4, 2, 580), (12, 1, 2, 600), (12, 4, 2, 1024), (12, 3, 2, 1025),
+                                     (8, 2, 300, 600), (12, 2, 700, 120), (5, 1, 3, 1024)])
+def test_viterbi_back_pointer_places_match_oracle(E, L, k, B, T):
+    """Paths on either side of where the targets are staged and the back-pointers lie: LDS where a row's fit and the rows
+    fit the chip together, the workspace otherwise, targets from memory past 1,024 positions."""
+    from lookatmyquant_amd.tables import quantile_table
+
+    tab = quantile_table(L, 0)
+    rng = np.random.default_rng(L * 1000 + T)
+    x = rng.standard_normal((B, T)).astype(np.float32)
+    st = rng.integers(0, 1 << L, B)
+    say(f"viterbi L={L} k={k} {B} x {T}")
+    got = E.viterbi_rows(cuda(x), cuda(tab.astype(np.float32)), L, k, start=cuda(st, torch.int32)).cpu().numpy()
+    pick = [0, B - 1]
+    assert np.array_equal(got[pick], O.viterbi(x[pick], tab, L, k, start=st[pick]))
+    free = E.viterbi_rows(cuda(x[:2]), cuda(tab.astype(np.float32)), L, k).cpu().numpy()
+    assert np.array_equal(free, O.viterbi(x[:2], tab, L, k))
+
+
 def test_viterbi_L16_long_paths_use_workspace(E):
     from lookatmyquant_amd.tables import quantile_table
 
