@@ -276,6 +276,117 @@ gemm128_f64_kernel(double* __restrict__ C, int64_t ldc, const double* __restrict
     cstore(3, g1);
 }
 
+// The same product on 64x64 tiles (four waves of 32x32 = 2x2 MFMA tiles), for shapes whose 128-tiles leave CUs idle: a
+// quarter of the tile gives four times the workgroups, whose 32 KB of LDS (two stage buffers of 16 in k) and registers
+// let four share a CU and cover each other's stage barriers. It reads its operands twice as often, 16 bytes a clock and
+// CU at the full MFMA rate, which L2 delivers. Layouts and swizzles as above, [row][k] rows of 128 bytes and [k][col]
+// rows of 64 columns.
+#define G6_BM 64
+#define G6_BK 16
+template <bool TRANSB, bool LOWER, int TRI = 0>
+__global__ __launch_bounds__(256, 4) void gemm64_f64_kernel(double* __restrict__ C, int64_t ldc,
+                                                            const double* __restrict__ A, int64_t lda,
+                                                            const double* __restrict__ B, int64_t ldb, int64_t M,
+                                                            int64_t N, int64_t K, const int32_t* __restrict__ info)
+{
+    constexpr int SB = G6_BM * G6_BK * 8;  // bytes of one operand stage
+    __shared__ __align__(16) uint8_t lds[2][2][SB];
+    if (info && *info != 0) return;
+    int64_t tr = (int64_t)blockIdx.y * G6_BM, tc = (int64_t)blockIdx.x * G6_BM;
+    if (TRI != 0) {  // the longest k-ranges first
+        const int64_t gx = gridDim.x, gy = gridDim.y, lin = (int64_t)blockIdx.y * gx + blockIdx.x;
+        const int64_t cr = lin / gy;
+        tr = (lin % gy) * G6_BM;
+        tc = (TRI == LAMQ_TRI_KGE ? cr : gx - 1 - cr) * G6_BM;
+    }
+    if (LOWER && tc > tr + G6_BM - 1) return;
+    const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
+    const int wr = (wave >> 1) * 32, wc = (wave & 1) * 32;
+    const int wv = __builtin_amdgcn_readfirstlane(wave);
+    const uint32_t base = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) uint8_t*)lds;
+    const double* zc = lamq_zero_chunk;
+    asm volatile("" : "+s"(zc));
+    // instruction i = 2 wv + q: eight rows of a [row][k] operand, two k-rows of a [k][col] one
+    auto load_rowk = [&](const double* X, int64_t ldx, int64_t r0, int64_t R, int64_t k0, int i, uint32_t m) {
+        const int r = 8 * i + lane / 8, c = (lane % 8) ^ ((r >> 1) & 7);
+        const int64_t row = r0 + r, k = k0 + 2 * c;
+        load_lds16(row < R && k < K ? X + row * ldx + k : zc, m);
+    };
+    auto load_kcol = [&](int64_t k0, int i, uint32_t m) {
+        const int kr = 2 * i + lane / 32, c = (lane % 32) ^ (8 * (kr & LAMQ_KSW_MASK));
+        const int64_t k = k0 + kr, col = tc + 2 * c;
+        load_lds16(k < K && col < N ? B + k * ldb + col : zc, m);
+    };
+    auto load_stage = [&](int64_t k0, int buf) {
+#pragma unroll
+        for (int q = 0; q < 2; ++q) {
+            const int i = 2 * wv + q;
+            load_rowk(A, lda, tr, M, k0, i, base + (uint32_t)(buf * 2 * SB + i * 1024));
+            if constexpr (TRANSB)
+                load_rowk(B, ldb, tc, N, k0, i, base + (uint32_t)((buf * 2 + 1) * SB + i * 1024));
+            else
+                load_kcol(k0, i, base + (uint32_t)((buf * 2 + 1) * SB + i * 1024));
+        }
+    };
+    const int li = lane & 15, lk = lane >> 4;
+    auto aaddr = [&](int row, int k) -> uint32_t {
+        return (uint32_t)(row * 128 + (((k >> 1) ^ ((row >> 1) & 7)) << 4) + (k & 1) * 8);
+    };
+    auto baddr = [&](int col, int k) -> uint32_t {
+        return TRANSB ? aaddr(col, k)
+                      : (uint32_t)(k * 512 + (((col >> 1) ^ (8 * (k & LAMQ_KSW_MASK))) << 4) + (col & 1) * 8);
+    };
+    lamq_d4 acc[2][2];
+#pragma unroll
+    for (int i = 0; i < 2; ++i)
+#pragma unroll
+        for (int j = 0; j < 2; ++j) acc[i][j] = lamq_d4{0.0, 0.0, 0.0, 0.0};
+    int st0 = 0, nst = (int)cdiv(K, G6_BK);
+    if (TRI == LAMQ_TRI_KGE) st0 = (int)(tc / G6_BK);
+    if (TRI == LAMQ_TRI_KLE && tc + G6_BM < K) nst = (int)cdiv(tc + G6_BM, G6_BK);
+    if (st0 < nst) load_stage((int64_t)st0 * G6_BK, st0 & 1);
+    for (int st = st0; st < nst; ++st) {
+        wait_vm<0>();     // this wave's loads of stage st have landed
+        __syncthreads();  // everyone's; the other buffer (stage st - 1) is free
+        if (st + 1 < nst) load_stage((int64_t)(st + 1) * G6_BK, (st + 1) & 1);
+        const uint8_t* As = lds[st & 1][0];
+        const uint8_t* Bs = lds[st & 1][1];
+#pragma unroll
+        for (int k4 = 0; k4 < G6_BK; k4 += 4) {
+            double a[2], b[2];
+#pragma unroll
+            for (int t = 0; t < 2; ++t) {
+                a[t] = *reinterpret_cast<const double*>(As + aaddr(wr + 16 * t + li, k4 + lk));
+                b[t] = *reinterpret_cast<const double*>(Bs + baddr(wc + 16 * t + li, k4 + lk));
+            }
+#pragma unroll
+            for (int i = 0; i < 2; ++i)
+#pragma unroll
+                for (int j = 0; j < 2; ++j) acc[i][j] = __builtin_amdgcn_mfma_f64_16x16x4f64(a[i], b[j], acc[i][j], 0, 0, 0);
+        }
+    }
+    // D layout (16x16): lane l, register v -> row 4*v + l/16, column l%16; every read of C before any write
+    double g[2][2][4];
+#pragma unroll
+    for (int i = 0; i < 2; ++i)
+#pragma unroll
+        for (int j = 0; j < 2; ++j)
+#pragma unroll
+            for (int v = 0; v < 4; ++v) {
+                const int64_t row = tr + wr + 16 * i + 4 * v + lk, col = tc + wc + 16 * j + li;
+                g[i][j][v] = (row < M && col < N && (!LOWER || col <= row)) ? C[row * ldc + col] : 0.0;
+            }
+#pragma unroll
+    for (int i = 0; i < 2; ++i)
+#pragma unroll
+        for (int j = 0; j < 2; ++j)
+#pragma unroll
+            for (int v = 0; v < 4; ++v) {
+                const int64_t row = tr + wr + 16 * i + 4 * v + lk, col = tc + wc + 16 * j + li;
+                if (row < M && col < N && (!LOWER || col <= row)) C[row * ldc + col] = g[i][j][v] - acc[i][j][v];
+            }
+}
+
 // Short products (K <= 128: the narrow refits of the sweep, the factor's panel products): the same C -= A op(B) (or
 // C = A op(B) with OVERWRITE) on 64x64 tiles whose whole k-range stays in LDS, in up to four stages of 32: every load
 // of every stage is issued at once (global_load_lds, 16 bytes a lane), and stage s is computed as soon as its own
@@ -520,6 +631,15 @@ __global__ __launch_bounds__(256) void gemm_splitk_f64_kernel(double* __restrict
 #define LAMQ_SPLITK_DEEPK 1024
 #endif
 
+// Deeper products whose 128-tiles (a LOWER one's: half of them) are fewer than this go out as 64-tiles. Measured, 128-tile
+// (or, under 128 tiles, the register kernel) against 64-tile: QEP's target (a factor and three products) of 1,024 x 2,560
+// (160 tiles) 2.87 -> 2.28 ms, 2,048 x 2,560 (320) 3.29 -> 2.63, 4,096 x 2,560 (640) 3.43 -> 3.29, 2,560 x 4,096 (640)
+// 6.53 -> 6.17; the factor at n = 1,024 / 2,560 / 4,096 655 -> 622, 1,718 -> 1,600, 3,165 -> 3,098 us. From 1,024 tiles
+// on the 128-tiles fill the chip and are ahead by up to 2% (4,096 x 4,096: 7.86 against 8.00 ms).
+#ifndef LAMQ_MID_TILES128
+#define LAMQ_MID_TILES128 1024
+#endif
+
 // TRI (LAMQ_TRI_KGE, LAMQ_TRI_KLE): op(B) is triangular and the 128-tile kernel skips the stages of its zero part (the
 // other kernels read the zeros).
 template <bool TRANSB, bool LOWER, bool OVERWRITE = false, int TRI = 0>
@@ -553,6 +673,15 @@ static int gemm_sub_f64(double* C, int64_t ldc, const double* A, int64_t lda, co
                                B, ldb, M, N, K, info);
         LAMQ_LAUNCH_CHECK();
         return LAMQ_OK;
+    }
+    if constexpr (!OVERWRITE) {
+        // (a LOWER product's 128-tiles: about half)
+        if (chunks && (LOWER ? tiles128 / 2 : tiles128) < LAMQ_MID_TILES128 && cdiv(M, 64) <= 65535) {
+            hipLaunchKernelGGL((gemm64_f64_kernel<TRANSB, LOWER, TRI>), grid, dim3(256), 0, s, C, ldc, A, lda, B, ldb, M, N,
+                               K, info);
+            LAMQ_LAUNCH_CHECK();
+            return LAMQ_OK;
+        }
     }
     if (!OVERWRITE && chunks && tiles128 >= 128) {
         dim3 grid128((unsigned)cdiv(N, G8_BM), (unsigned)cdiv(M, G8_BM));

@@ -276,6 +276,27 @@ def test_gemm_sub_short_k(E, M, N, K, transb):
     assert err < 1e-13
 
 
+@pytest.mark.parametrize("M,N,K,transb,tri", [(65, 130, 1026, False, 0), (64, 64, 1040, True, 0), (1, 2, 130, True, 0),
+                                              (700, 1300, 1300, True, 1), (129, 1298, 1298, False, 2),
+                                              (63, 1100, 1100, False, 1), (1000, 1026, 1026, True, 2),
+                                              (3970, 4034, 144, True, 0)])
+def test_gemm_sub_64_tiles(E, M, N, K, transb, tri):
+    """Deep products whose 128-tiles are too few for the chip, on the 64-tile streaming kernel: ragged M, N and K, both
+    layouts and both triangular forms, C a slice of a wider matrix whose other columns stay as they are, against a
+    float64 product on the GPU."""
+    g = torch.Generator(device="cuda").manual_seed(M + 3 * N + 7 * K + tri)
+    Cw = torch.randn(M, N + 6, generator=g, device="cuda", dtype=torch.float64)
+    A = torch.randn(M, K, generator=g, device="cuda", dtype=torch.float64)
+    opB = torch.randn(K, N, generator=g, device="cuda", dtype=torch.float64)
+    opB = torch.tril(opB) if tri == 1 else torch.triu(opB) if tri == 2 else opB
+    ref = Cw.clone()
+    ref[:, 2 : 2 + N] -= A @ opB
+    say(f"gemm_sub 64-tile: M={M} N={N} K={K} transb={transb} tri={tri}")
+    E.gemm_sub(Cw[:, 2 : 2 + N], A, (opB.T if transb else opB).contiguous(), transb=transb, tri=tri)
+    err = ((Cw - ref).abs().max() / ref.abs().max()).item()
+    assert err < 1e-13
+
+
 @pytest.mark.parametrize("M,N,K", [(2560, 9216, 512), (2560, 1536, 512), (6144, 1536, 512), (19456, 2048, 512),
                                    (300, 1000, 136), (2560, 3584, 512), (2500, 700, 512), (77, 130, 1024),
                                    (2560, 128, 512)])
