@@ -264,6 +264,10 @@ int lamq_rht_rows(const double* in, int64_t rows, int64_t n, int64_t ldi, double
  * return LAMQ_EUNSUP (lamq_rht_rows takes them). The results differ from lamq_rht_rows's in float64 rounding only. */
 int lamq_rht_rows_sylvester(const double* in, int64_t rows, int64_t n, int64_t ldi, double* out, int64_t ldo,
                             const int8_t* signs, int b, int inverse, double* rms, void* stream);
+int lamq_transpose_f64(const double* in, int64_t rows, int64_t cols, int64_t ldi, double* out, int64_t ldo,
+                       void* stream);
+/* Row scales S_r = max(sqrt(mean_j X[r, j]^2), 1e-12) (opgraph/codes.py:436, nested.py:168). */
+int lamq_row_rms(const double* X, int64_t rows, int64_t n, int64_t ldx, double* S, void* stream);
 
 /* ------------------------------------------------------------------------------------------------
  * Token-weighted Gram matrix on bf16 MFMA with fp32 accumulation:

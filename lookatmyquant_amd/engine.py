@@ -23,7 +23,7 @@ class LinAlgError(torch.linalg.LinAlgError if hasattr(torch.linalg, "LinAlgError
 # ----------------------------------------------------------------------------- Viterbi (codes.py:151-181)
 
 
-BIG_L = 13  # tables of 2^13 states and more go to the 1024-thread kernels (fp16-exact tables)
+BIG_L = 13  # tables of 2^13 states and more go to the 16-bit-state kernels (fp16-exact tables)
 MERGED_SMALL_L = 12  # below BIG_L, the state width whose row groups go through one launch per lazy block
 
 
