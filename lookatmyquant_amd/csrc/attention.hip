@@ -36,6 +36,7 @@
 typedef __bf16 lamq_at_bf16x8 __attribute__((ext_vector_type(8)));
 typedef float lamq_at_f32x16 __attribute__((ext_vector_type(16)));
 
+#define AT_GRID_X (1 << 22)
 #define AT_D 128                        // head dim
 #define AT_QW 32                        // queries per wave
 #define AT_KB 32                        // keys per half block (one S^T tile)
@@ -78,7 +79,8 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
     // workgroup -> (pair of sequence and key/value head, query head of the pair, query block)
     int pair, rem;
     {
-        const int id = (int)blockIdx.x, per = nqb * rep;
+        const int id = (int)(blockIdx.y * gridDim.x + blockIdx.x), per = nqb * rep;
+        if ((unsigned)id >= (unsigned)pairs * (unsigned)per) return;  // past the last (the grid's last row)
         if (pairs % LAMQ_XCDS == 0) {
             const int y = id / LAMQ_XCDS;
             pair = y / per * LAMQ_XCDS + id % LAMQ_XCDS;
@@ -277,9 +279,12 @@ extern "C" int lamq_attention_causal_bf16(const uint16_t* q, int64_t sqb, int64_
     if (B == 0 || T == 0) return LAMQ_OK;
     if (B > 65535 || H > 65535 || T > 0x7fffff) return LAMQ_EUNSUP;
     if (cdiv(T, AT_QB) * H * B > 0x7fffffff) return LAMQ_EUNSUP;
-    const dim3 grid((unsigned)(cdiv(T, AT_QB) * H * B));
+    // a grid's work items along x must stay below 2^32, so past 2^22 workgroups they go out in rows
+    const int64_t wgs = cdiv(T, AT_QB) * H * B, gx = wgs < AT_GRID_X ? wgs : AT_GRID_X;
+    const dim3 grid((unsigned)gx, (unsigned)cdiv(wgs, gx));
     hipLaunchKernelGGL(attention_causal_kernel, grid, dim3(256), 0, as_stream(stream), q, sqb, sqh, sqt, k, skb, skh, skt,
-                       v, svb, svh, svt, out, sob, soh, sot, (int)(H / Hkv), (int)Hkv, (int)(B * Hkv), (int)T, scale * 1.4426950408889634f);
+                       v, svb, svh, svt, out, sob, soh, sot, (int)(H / Hkv), (int)Hkv, (int)(B * Hkv), (int)T,
+                       scale * 1.4426950408889634f);
     LAMQ_LAUNCH_CHECK();
     return LAMQ_OK;
 }

@@ -709,6 +709,7 @@ __global__ __launch_bounds__((B * (1 << K) / 16 + 63) / 64 * 64) void rht_paley_
     if (rms) rht_row_rms(ss, part, NT, N, rms + blockIdx.x);
 }
 
+#define RHT_ROWS_MAX ((int64_t)1 << 22)
 extern "C" int lamq_rht_rows_sylvester(const double* in, int64_t rows, int64_t n, int64_t ldi, double* out, int64_t ldo,
                                        const int8_t* signs, int b, int inverse, double* rms, void* stream)
 {
@@ -721,6 +722,14 @@ extern "C" int lamq_rht_rows_sylvester(const double* in, int64_t rows, int64_t n
     const bool ok = b == 1 ? (k >= 10 && k <= 13) : ((b == 12 || b == 20) && k >= 4 && k <= 8);
     if (!ok) return LAMQ_EUNSUP;
     if (rows == 0) return LAMQ_OK;
+    if (rows > RHT_ROWS_MAX) {  // a grid's work items along x must stay below 2^32
+        for (int64_t r = 0; r < rows; r += RHT_ROWS_MAX) {
+            const int e = lamq_rht_rows_sylvester(in + r * ldi, rows - r < RHT_ROWS_MAX ? rows - r : RHT_ROWS_MAX, n, ldi,
+                                                  out + r * ldo, ldo, signs, b, inverse, rms ? rms + r : nullptr, stream);
+            if (e != LAMQ_OK) return e;
+        }
+        return LAMQ_OK;
+    }
     const dim3 grid((unsigned)rows);
     hipStream_t s = as_stream(stream);
     const double sqrt_n = sqrt((double)n);

@@ -192,6 +192,18 @@ def test_fused_attention_growing_scores_and_edges(B, H, Hkv, T, trend):
     assert bool(((got - P @ vv).abs() <= 2.0 ** -7 * (P @ vv.abs())).all())
 
 
+def test_fused_attention_past_a_grid_row():
+    """More workgroups than one row of the grid holds (2^22), the last row partly past the end: one-token sequences, each
+    output its v."""
+    from lookatmyquant_amd import engine as E
+
+    B, H = 65535, 65
+    v = torch.randn(B, 1, 1, 128, device="cuda").bfloat16()
+    q = torch.ones(1, 1, 1, 128, device="cuda", dtype=torch.bfloat16).expand(B, H, 1, 128)
+    got = E.attention_causal(q, v, v, 0.1)
+    assert bool((got == v).all())
+
+
 @pytest.mark.parametrize("B,H,Hkv,T", [(2, 32, 8, 2048), (3, 4, 4, 33), (1, 8, 2, 1)])
 def test_fused_attention_shapes_against_float64(B, H, Hkv, T):
     """The fused attention at the config-5 shape (GQA 32/8, T = 2,048), a ragged T with one query block partly past it
