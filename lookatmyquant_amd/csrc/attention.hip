@@ -232,15 +232,17 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
         lrun += (ps[0] + ps[1]) + (ps[2] + ps[3]);
 #pragma unroll
         for (int hf = 0; hf < 2; ++hf)
+            // uniform; a half past the wave's last query has no part in the sums (32 heads x 333: 14.9 -> 14.4 us)
+            if (hf == 0 || k0 + AT_KB <= my_last)
 #pragma unroll
-            for (int mi = 0; mi < 2; ++mi)
+                for (int mi = 0; mi < 2; ++mi)
 #pragma unroll
-                for (int t = 0; t < 4; ++t) {
-                    const short __attribute__((ext_vector_type(8))) w =
-                        __builtin_shufflevector(vf[hf][t][mi][0], vf[hf][t][mi][1], 0, 1, 2, 3, 4, 5, 6, 7);
-                    o[t] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(lamq_at_bf16x8, w), pf[hf][mi], o[t],
-                                                                   0, 0, 0);
-                }
+                    for (int t = 0; t < 4; ++t) {
+                        const short __attribute__((ext_vector_type(8))) w =
+                            __builtin_shufflevector(vf[hf][t][mi][0], vf[hf][t][mi][1], 0, 1, 2, 3, 4, 5, 6, 7);
+                        o[t] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(lamq_at_bf16x8, w), pf[hf][mi],
+                                                                       o[t], 0, 0, 0);
+                    }
         // the next iteration's barrier comes after every wave's reads of this buffer (their results are used above)
     }
     if (myq >= T) return;

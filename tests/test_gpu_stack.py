@@ -192,6 +192,17 @@ def test_fused_attention_growing_scores_and_edges(B, H, Hkv, T, trend):
     assert bool(((got - P @ vv).abs() <= 2.0 ** -7 * (P @ vv.abs())).all())
 
 
+def test_fused_attention_leaves_out_values_past_a_waves_queries():
+    """The first 32 queries of a block of 64 keys share a wave that no value past key 31 enters, not even as 0 x NaN."""
+    from lookatmyquant_amd import engine as E
+
+    g = torch.Generator(device="cuda").manual_seed(3)
+    q, k, v = (torch.randn(1, 2, 50, 128, generator=g, device="cuda").bfloat16() for _ in range(3))
+    ref = E.attention_causal(q[:, :, :32], k[:, :, :32], v[:, :, :32], 128 ** -0.5)
+    v[:, :, 32:] = float("nan")
+    assert torch.equal(E.attention_causal(q, k, v, 128 ** -0.5)[:, :, :32], ref)
+
+
 def test_fused_attention_past_a_grid_row():
     """More workgroups than one row of the grid holds (2^22), the last row partly past the end: one-token sequences, each
     output its v."""
