@@ -22,17 +22,23 @@
 // one to LDS. 256 paths of 256 positions at L = 12 (one a CU), k = 1 .. 4: 109, 99, 114 and 122 us with both in memory,
 // 110, 99, 106 and 117 with the targets staged, 96, 92, 89 and 104 with the back-pointers in LDS too.
 #define LAMQ_TV_STAGE 1024
-template <int L, int K, bool BACK_GLOBAL, bool STAGE>
-__global__ __launch_bounds__(LAMQ_NT) void viterbi_rows_kernel(const float* __restrict__ x, int T, int64_t ldx,
+// Where the rows are no more than the CUs, a row has one wave a SIMD and its steps wait on their own barrier and LDS round
+// trip; on 512 threads, half the groups each, two waves cover each other. 256 x 256 at L = 12, k = 1, 2, 3: 82.0, 77.6
+// and 76.0 -> 71.0, 65.0 and 71.0 us; 64 x 32 12.3, 11.7, 11.6 -> 10.8, 10.3, 10.8. Not with two rows a CU (512 x 64:
+// 24.4, 22.3, 22.2 us on 256 threads, 23.8, 22.1, 23.7 on 512) nor for short paths (256 x 8: 6.5 -> 6.7 us).
+#define LAMQ_TV_WIDE 512
+#define LAMQ_TV_WIDE_MIN 32  // shortest path on LAMQ_TV_WIDE threads
+template <int L, int K, bool BACK_GLOBAL, bool STAGE, int NT = LAMQ_NT>
+__global__ __launch_bounds__(NT) void viterbi_rows_kernel(const float* __restrict__ x, int T, int64_t ldx,
                                                                const float* __restrict__ C,
                                                                const int32_t* __restrict__ start,
                                                                int32_t* __restrict__ states, int64_t lds,
                                                                uint8_t* __restrict__ back_ws)
 {
-    using V = VX<L, K, LAMQ_NT>;
+    using V = VX<L, K, NT>;
     extern __shared__ __align__(16) float dyn[];  // STAGE: T targets (to 16 bytes); then the back-pointers in LDS
     __shared__ __align__(16) float buf[2 * V::R];
-    __shared__ __align__(8) float red[2 * (LAMQ_NT / 64)];
+    __shared__ __align__(8) float red[2 * (NT / 64)];
     const int64_t row = blockIdx.x;
     const int tid = threadIdx.x;
     TabF32<V> tab;
@@ -40,16 +46,16 @@ __global__ __launch_bounds__(LAMQ_NT) void viterbi_rows_kernel(const float* __re
     const float* xr = x + row * ldx;
     const int st = start ? start[row] : -1;
     if constexpr (STAGE) {
-        for (int t = tid; t < T; t += LAMQ_NT) dyn[t] = search_target(xr[t]);
+        for (int t = tid; t < T; t += NT) dyn[t] = search_target(xr[t]);
         __syncthreads();
         if constexpr (BACK_GLOBAL)
-            viterbi_gx<L, K, LAMQ_NT, true, true>(dyn, T, tab, st, buf, back_ws + row * (int64_t)(T - 1) * V::ACT,
+            viterbi_gx<L, K, NT, true, true>(dyn, T, tab, st, buf, back_ws + row * (int64_t)(T - 1) * V::ACT,
                                                   states + row * lds, red);
         else
-            viterbi_gx<L, K, LAMQ_NT, true, false>(dyn, T, tab, st, buf, reinterpret_cast<uint8_t*>(dyn + (T + 3) / 4 * 4),
+            viterbi_gx<L, K, NT, true, false>(dyn, T, tab, st, buf, reinterpret_cast<uint8_t*>(dyn + (T + 3) / 4 * 4),
                                                    states + row * lds, red);
     } else {
-        viterbi_gx<L, K, LAMQ_NT, true, true, false, true>(xr, T, tab, st, buf, back_ws + row * (int64_t)(T - 1) * V::ACT,
+        viterbi_gx<L, K, NT, true, true, false, true>(xr, T, tab, st, buf, back_ws + row * (int64_t)(T - 1) * V::ACT,
                                                            states + row * lds, red);
     }
 }
@@ -64,6 +70,20 @@ struct ViterbiRows {
         constexpr int64_t CUS = 256;
         const size_t need = T <= LAMQ_TV_LDS ? 0 : (size_t)B * (size_t)T * V::ACT;
         if (need && (!ws || ws_bytes < need)) return LAMQ_EINVAL;
+        if constexpr (V::R >= LAMQ_TV_WIDE) {
+            using W = VX<L, K, LAMQ_TV_WIDE>;
+            constexpr size_t WFIXED = 4 * 2 * W::R + 4 * 2 * (LAMQ_TV_WIDE / 64);
+            const size_t dynb = 16 * ((size_t)(T + 3) / 4) + (size_t)(T - 1) * W::ACT;
+            if (B <= CUS && T >= LAMQ_TV_WIDE_MIN && T <= LAMQ_TV_STAGE && WFIXED + dynb <= CU_LDS) {
+                if (WFIXED + dynb > 48 * 1024)
+                    LAMQ_HIP_CHECK(hipFuncSetAttribute((const void*)viterbi_rows_kernel<L, K, false, true, LAMQ_TV_WIDE>,
+                                                       hipFuncAttributeMaxDynamicSharedMemorySize, (int)(CU_LDS - WFIXED)));
+                hipLaunchKernelGGL((viterbi_rows_kernel<L, K, false, true, LAMQ_TV_WIDE>), dim3((unsigned)B),
+                                   dim3(LAMQ_TV_WIDE), dynb, s, x, T, ldx, C, start, states, lds, (uint8_t*)nullptr);
+                LAMQ_LAUNCH_CHECK();
+                return LAMQ_OK;
+            }
+        }
         const size_t xb = 16 * ((size_t)(T + 3) / 4), bb = (size_t)(T - 1) * V::ACT;
         const bool fits = FIXED + xb + bb <= CU_LDS;
         if (T <= LAMQ_TV_LDS ||

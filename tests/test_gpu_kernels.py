@@ -156,6 +156,24 @@ def test_viterbi_back_pointer_places_match_oracle(E, L, k, B, T):
     assert np.array_equal(free, O.viterbi(x[:2], tab, L, k))
 
 
+@pytest.mark.parametrize("L,k,B,T", [(12, 2, 2, 31), (12, 1, 256, 32), (12, 3, 257, 32), (12, 2, 3, 301), (12, 2, 3, 303),
+                                     (12, 3, 2, 45), (11, 2, 5, 64), (10, 1, 4, 33), (10, 2, 4, 33)])
+def test_viterbi_wide_rows_match_oracle(E, L, k, B, T):
+    """Either side of where a row takes 512 threads: path length, row count, LDS, and at least 512 groups."""
+    from lookatmyquant_amd.tables import quantile_table
+
+    tab = quantile_table(L, 0)
+    rng = np.random.default_rng(L * 1000 + T + k)
+    x = rng.standard_normal((B, T)).astype(np.float32)
+    st = rng.integers(0, 1 << L, B)
+    say(f"viterbi L={L} k={k} {B} x {T}")
+    pick = [0, B - 1]
+    for start in (None, st):
+        sg = None if start is None else cuda(start, torch.int32)
+        got = E.viterbi_rows(cuda(x), cuda(tab.astype(np.float32)), L, k, start=sg).cpu().numpy()
+        assert np.array_equal(got[pick], O.viterbi(x[pick], tab, L, k, start=None if start is None else start[pick]))
+
+
 def test_viterbi_L16_long_paths_use_workspace(E):
     from lookatmyquant_amd.tables import quantile_table
 
