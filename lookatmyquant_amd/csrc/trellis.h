@@ -355,9 +355,12 @@ __device__ int viterbi_gx(const float* xs, int TV, Tab& tab, int start, float* b
     const bool act = V::ACT >= NT || tid < V::ACT;
     // groups stored together: those sharing one B entry per h, and four at least
     constexpr int CK = V::RUN ? (NB < 4 && G >= 4 ? 4 : NB) : G;
+    // Fewer groups than members of one (L < 2K, one group a thread): (h*R + tid) >> K is (h*R) >> K for every tid < R, the
+    // same entry for the 2^(2K-L) members h of a run and for every thread.
+    constexpr bool FEW = R < NB;
     int ent[NB];
 #pragma unroll
-    for (int h = 0; h < NB; ++h) ent[h] = V::RUN ? h * (R >> K) + M * tid : (h * R + G * tid) >> K;
+    for (int h = 0; h < NB; ++h) ent[h] = FEW ? (h * R) >> K : V::RUN ? h * (R >> K) + M * tid : (h * R + G * tid) >> K;
     float bv[NB][M];
     // ent[h] = ent[0] + h (R >> K) where R is a multiple of 2^K; a stride the swizzle keeps (swz(x + d) = swz(x) + d)
     // then makes one swizzled index serve every h
@@ -372,11 +375,12 @@ __device__ int viterbi_gx(const float* xs, int TV, Tab& tab, int start, float* b
     // the group minima before position 0: 0 for the start's group (every group with a free start), else +inf
     const auto start_minima = [&]() {
         const int rs = start >= 0 ? (start & (R - 1)) : -1;
-        const int d = rs - ent[0];  // ent[h] + e == rs exactly when d == h (R >> K) + e
+        const int d = rs - ent[0];  // ent[h] + e == rs exactly when d == h (R >> K) + e (with FEW: when d == ent[h])
 #pragma unroll
         for (int h = 0; h < NB; ++h)
 #pragma unroll
-            for (int e = 0; e < M; ++e) bv[h][e] = (rs < 0 || d == h * (R >> K) + e) ? 0.0f : __builtin_inff();
+            for (int e = 0; e < M; ++e)
+                bv[h][e] = (rs < 0 || d == (FEW ? ent[h] : h * (R >> K)) + e) ? 0.0f : __builtin_inff();
     };
     // (a thread of many states has no registers to spare for sixteen of them: two halves of eight)
     constexpr int NLO = NB == 16 && V::SPT > 64 ? 8 : NB;

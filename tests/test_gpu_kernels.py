@@ -174,6 +174,31 @@ def test_viterbi_wide_rows_match_oracle(E, L, k, B, T):
         assert np.array_equal(got[pick], O.viterbi(x[pick], tab, L, k, start=None if start is None else start[pick]))
 
 
+@pytest.mark.parametrize("L,k", [(3, 2), (4, 3), (5, 3), (5, 4), (6, 4), (7, 4), (2, 1), (4, 2), (6, 3), (8, 4)])
+def test_fewer_groups_than_members_matches_oracle(E, L, k):
+    """2^(L-k) groups of 2^k members with L < 2k (and L = 2k beside it), a fixed and a free first state: the standalone
+    search and the fused sweep, whose every search but the first starts where the one before ended."""
+    from lookatmyquant_amd.tables import quantile_table
+
+    tab = quantile_table(L, 0)
+    rng = np.random.default_rng(50 * L + k)
+    n = 72
+    Xa = rng.standard_normal((3 * n, n))
+    _, U, _ = O.environment(Xa.T @ Xa / (3 * n))
+    for B, T in ((5, 9), (300, 70)):
+        x = rng.standard_normal((B, T)).astype(np.float32)
+        for start in (None, rng.integers(0, 1 << L, B)):
+            say(f"viterbi L={L} k={k} {B} x {T}")
+            sg = None if start is None else cuda(start, torch.int32)
+            got = E.viterbi_rows(cuda(x), cuda(tab.astype(np.float32)), L, k, start=sg).cpu().numpy()
+            assert np.array_equal(got, O.viterbi(x, tab, L, k, start=start))
+    X = rng.standard_normal((9, n))
+    S = O.row_scale(X)
+    say(f"ldlq trellis L={L} k={k}")
+    got = E.ldlq_trellis(cuda(X), cuda(S), cuda(U), cuda(tab), L, k).cpu().numpy()
+    assert np.array_equal(got, O.ldlq_trellis(X, U, S, tab, L, k))
+
+
 def test_viterbi_L16_long_paths_use_workspace(E):
     from lookatmyquant_amd.tables import quantile_table
 
