@@ -5,18 +5,21 @@
 // (global_load_lds, 16 bytes a lane, no registers), double-buffered, the next block's loads issued as soon as the
 // current one is published (one barrier a block), so the four waves share one copy and no wave waits on a global
 // load. Per block a wave forms S^T = K Q^T (two tiles of 32 keys x 32 queries: the head dim, 128, as eight 16-deep steps of
-// v_mfma_f32_32x32x16_bf16 each, float32 sums), masks it where the block reaches past its first query, updates each
-// query's maximum and its lanes' parts of the sum (the online softmax: exp2 with the scale and log2(e) folded into one
-// multiply-add a score), rounds the probabilities to bf16 and accumulates O^T += V^T P^T (128 x 32, float32); a wave past
-// its own last query skips the block (which still arrives for the others). At the end O = O^T / sum, rounded to bf16
-// (nearest, ties to even).
+// v_mfma_f32_32x32x16_bf16 each, float32 sums) and masks it where the block reaches past its first query; then, half by
+// half of 32 keys, it updates each query's running maximum and sum (the online softmax: exp2 with the scale and log2(e)
+// folded into the scores), rounds the probabilities to bf16 and accumulates O^T += V^T P^T (128 x 32, float32); a wave
+// past its own last query skips the half (whose block still arrives for the others). At the end O = O^T / sum, rounded
+// to bf16 (nearest, ties to even).
 //
 // What bounds it: with two waves a SIMD the vector work of one runs under the matrix work of the other, 1,024 clocks a
-// block, so the vector chain of a block is kept short: 64 keys a softmax instead of 32, no mask off the diagonal, the
-// earlier sums rescaled only when some query's maximum has grown (a lag of 2^8 allowed would save 5%, but the largest
-// probability is then no longer exactly 1 before its rounding to bf16), the halves of a query's keys combined by a swap of the wave's halves (LDS shuffles
-// before) and its sum only at the end, row pointers advanced a block at a time, and V's transposing reads issued before
-// the softmax they are needed after. 8 x 32 heads x 2,048: 655 -> 330 us (833 TFLOP/s); 32 sequences 2.56 -> 1.29 ms.
+// block, so the vector chain of a block is kept short: both halves' scores and maxima at once, no mask off the diagonal,
+// the earlier sums rescaled only when some query's maximum has grown, the lanes of a query's keys combined by a swap of
+// the wave's halves (LDS shuffles before), row pointers advanced a block at a time, and V's transposing reads issued
+// before the softmax they are needed after. The results are those of 32 keys at a time, bit for bit: one softmax step
+// for all 64 keys, its scale folded into a multiply-add, is another 7% faster, but a probability of the first half is
+// then rounded to bf16 under a maximum it has not met (relative error against float64 of the 8-sequence case 2.01e-3
+// -> 2.02e-3). 8 x 32 heads x 2,048: 657 -> 370-385 us (715-745 TFLOP/s); 32 sequences 2.59 -> 1.40 ms; one of 333
+// tokens 14.9 -> 12.9 us.
 // Workgroups go out pair by pair of sequence and key/value head, pairs spread over the XCDs, so that the query heads and
 // blocks that read the same K and V run on one XCD together.
 //
@@ -153,7 +156,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
     for (int t = 0; t < 4; ++t)
 #pragma unroll
         for (int v = 0; v < 16; ++v) o[t][v] = 0.0f;
-    float mrun = -__builtin_inff(), lrun = 0.0f;  // the maximum (of the scaled scores), this lane's part of the sum
+    float mrun = -__builtin_inff(), lrun = 0.0f;  // each query's maximum (of the scaled scores) and sum
     for (int kb = 0; kb < nblk; ++kb) {
         wait_vm<0>();     // this wave's loads of block kb have landed
         __syncthreads();  // everyone's; the other buffer (block kb - 1) is free
@@ -204,49 +207,54 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
                     s[hf][v] = key <= myq ? s[hf][v] : -__builtin_inff();
                 }
         }
-        float mx = fmaxf(s[0][0], s[1][0]);
+        // the running maximum after each half's 32 keys (finite from the first half on: key 0 is never masked). The scale
+        // is positive and its product rounded monotonically, so the scaled maximum is the maximum of the scaled scores
+        float m[2];
 #pragma unroll
-        for (int v = 1; v < 16; ++v) mx = fmaxf(fmaxf(mx, s[0][v]), s[1][v]);
-        const float ms = at_max32(mx) * scale_log2;
-        // the sums are rescaled only in blocks where some query's maximum grows
-        if (__builtin_amdgcn_ballot_w64(ms > mrun)) {
-            const float mnew = fmaxf(mrun, ms);  // finite from the first block on: key 0 is never masked
-            const float alpha = __builtin_amdgcn_exp2f(mrun - mnew);  // 0 on the first block
-            lrun *= alpha;
-            mrun = mnew;
+        for (int hf = 0; hf < 2; ++hf) {
+            float mx = s[hf][0];
 #pragma unroll
-            for (int t = 0; t < 4; ++t)
-#pragma unroll
-                for (int v = 0; v < 16; ++v) o[t][v] *= alpha;
+            for (int v = 1; v < 16; ++v) mx = fmaxf(mx, s[hf][v]);
+            m[hf] = fmaxf(hf == 0 ? mrun : m[0], at_max32(mx) * scale_log2);
         }
-        lamq_at_bf16x8 pf[2][2];
-        float ps[4] = {0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll
         for (int hf = 0; hf < 2; ++hf)
+            // uniform; a half past the wave's last query has no part in the sums
+            if (hf == 0 || k0 + AT_KB <= my_last) {
+                lamq_at_bf16x8 pf[2];
+                float ps = 0.0f;
 #pragma unroll
-            for (int v = 0; v < 16; ++v) {
-                const float p = __builtin_amdgcn_exp2f(fmaf(s[hf][v], scale_log2, -mrun));  // masked: exp2(-inf) = 0
-                ps[v & 3] += p;
-                pf[hf][v >> 3][v & 7] = (__bf16)p;
-            }
-        lrun += (ps[0] + ps[1]) + (ps[2] + ps[3]);
+                for (int v = 0; v < 16; ++v) {
+                    const float x = s[hf][v] * scale_log2;
+                    const float p = __builtin_amdgcn_exp2f(x - m[hf]);  // masked: exp2(-inf) = 0
+                    ps += p;
+                    pf[v >> 3][v & 7] = (__bf16)p;
+                }
+                // the sums are rescaled only in halves where some query's maximum grows (elsewhere by exactly 1)
+                if (__builtin_amdgcn_ballot_w64(m[hf] > mrun)) {
+                    const float alpha = __builtin_amdgcn_exp2f(mrun - m[hf]);  // 0 on the first half
+                    lrun *= alpha;
+                    mrun = m[hf];
 #pragma unroll
-        for (int hf = 0; hf < 2; ++hf)
-            // uniform; a half past the wave's last query has no part in the sums (32 heads x 333: 14.9 -> 14.4 us)
-            if (hf == 0 || k0 + AT_KB <= my_last)
+                    for (int t = 0; t < 4; ++t)
+#pragma unroll
+                        for (int v = 0; v < 16; ++v) o[t][v] *= alpha;
+                }
+                lrun += at_sum32(ps);
 #pragma unroll
                 for (int mi = 0; mi < 2; ++mi)
 #pragma unroll
                     for (int t = 0; t < 4; ++t) {
                         const short __attribute__((ext_vector_type(8))) w =
                             __builtin_shufflevector(vf[hf][t][mi][0], vf[hf][t][mi][1], 0, 1, 2, 3, 4, 5, 6, 7);
-                        o[t] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(lamq_at_bf16x8, w), pf[hf][mi],
+                        o[t] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(lamq_at_bf16x8, w), pf[mi],
                                                                        o[t], 0, 0, 0);
                     }
+            }
         // the next iteration's barrier comes after every wave's reads of this buffer (their results are used above)
     }
     if (myq >= T) return;
-    const float inv = 1.0f / at_sum32(lrun);
+    const float inv = 1.0f / lrun;
     uint16_t* Op = O + b * sob + (int64_t)h * soh + (int64_t)myq * sot;
 #pragma unroll
     for (int t = 0; t < 4; ++t)

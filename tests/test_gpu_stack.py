@@ -192,6 +192,29 @@ def test_fused_attention_growing_scores_and_edges(B, H, Hkv, T, trend):
     assert bool(((got - P @ vv).abs() <= 2.0 ** -7 * (P @ vv.abs())).all())
 
 
+def test_fused_attention_rounds_a_half_block_under_its_own_maximum():
+    """Keys 0-31 all score 0 and keys 32-63 all score c > 0. The probabilities of each half, taken under the running maximum
+    after that half's 32 keys, are then exactly 1, and the first half's sums are rescaled in float32: the only bf16
+    rounding left is the result's. Bound: half a bf16 spacing of the exact value, and 2^-18 of it for the float32
+    sums, product and exponential."""
+    from lookatmyquant_amd import engine as E
+
+    H, T = 32, 64
+    c = torch.linspace(0.05, 6.0, H, device="cuda").bfloat16()
+    q = torch.zeros(1, H, T, 128, device="cuda", dtype=torch.bfloat16)
+    k, v = torch.zeros_like(q), torch.zeros_like(q)
+    q[..., 0] = 1.0
+    k[:, :, 32:, 0] = c[None, :, None]
+    v[:, :, :32, 0] = 1.0
+    v[:, :, 32:, 1] = 1.0
+    got = E.attention_causal(q, k, v, 1.0)[0, :, 32:, :2].double().cpu()
+    a = 32.0 * torch.exp(-c.double().cpu())[:, None]
+    n = torch.arange(1, 33, dtype=torch.float64)[None, :]
+    want = torch.stack([a / (a + n), n / (a + n)], -1)
+    half_spacing = 2.0 ** (torch.floor(torch.log2(want)) - 8)
+    assert bool(((got - want).abs() <= half_spacing + 2.0 ** -18 * want).all())
+
+
 def test_fused_attention_leaves_out_values_past_a_waves_queries():
     """The first 32 queries of a block of 64 keys share a wave that no value past key 31 enters, not even as 0 x NaN."""
     from lookatmyquant_amd import engine as E
