@@ -27,8 +27,9 @@ FLAGS = ["-O3", "-fPIC", "-std=c++17", f"--offload-arch={ARCH}", "-ffp-contract=
 # Per-file additions. The fp64 MFMA kernels keep their accumulators in VGPR-form MFMAs (-amdgpu-mfma-vgpr-form): left
 # to itself, the register allocator carries them around the k-loop in VGPRs and copies them into AGPRs every stage,
 # and AGPR-form f64 MFMAs measured at half the rate of VGPR-form ones (34.7 against 68.6 TFLOP/s on a pure MFMA loop).
-# The trellis searches never produce a NaN (costs are finite or +inf, and inf - inf never forms), so they are
-# built with -fno-honor-nans: a minimum is then one v_min (f32 or f64), with no canonicalising of its operands first.
+# The trellis searches never hold a NaN (a NaN target enters as +inf, search_target; tables are finite, so costs are finite
+# or +inf, and inf - inf never forms), so they are built with -fno-honor-nans: a minimum is then one v_min (f32 or f64),
+# with no canonicalising of its operands first.
 FILE_FLAGS = {"ldlq.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form=1"], "chol.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form=1"],
               "rht.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form=1"],
               "viterbi.hip": ["-fno-honor-nans"], "viterbi16.hip": ["-fno-honor-nans"]}

@@ -177,14 +177,16 @@ __device__ __forceinline__ double cost_and(float c, uint32_t lo) { return __hilo
 __device__ __forceinline__ float cost_of(double p) { return __int_as_float(__double2hiint(p)); }
 __device__ __forceinline__ uint32_t low_of(double p) { return (uint32_t)__double2loint(p); }
 
-// A target as the searches take it: a NaN with its sign cleared, so that the costs it makes are positive NaNs, above every
-// other pair, and an all-NaN group keeps its lowest h (a comparison, which no NaN wins, would too). On the bits, made
-// opaque: the searches are compiled without NaNs, and the compiler would take the test for one and drop it.
+// A target as the searches take it: a NaN as +inf. Either makes every cost of its position and of all later ones compare
+// alike (no NaN wins a comparison, and the +inf all tie), so every group keeps its lowest h, the path ends in state 0 and
+// the states are the same; but no NaN ever forms (the tables are finite and inf - inf never arises), which the searches
+// are compiled to rely on. On the bits, made opaque: the compiler would take a test of the float for one on a NaN that
+// cannot be, and drop it.
 __device__ __forceinline__ float search_target(float x)
 {
     uint32_t b = (uint32_t)__float_as_int(x);
     asm volatile("" : "+v"(b));
-    return __int_as_float((int)((b & 0x7FFFFFFFu) > 0x7F800000u ? 0x7FC00000u : b));
+    return __int_as_float((int)((b & 0x7FFFFFFFu) > 0x7F800000u ? 0x7F800000u : b));
 }
 
 template <int N>
@@ -340,7 +342,7 @@ __device__ __forceinline__ int wave_imin(int v)
 // or writes buf any more.
 template <int L, int K, int NT, bool DBL, bool BACK_GLOBAL = false, bool PATHREG = false, bool RAWX = false,
           typename BackT, class Tab, class Hook = NoHook, class BufHook = NoHook>
-__device__ int viterbi_gx(const float* xs, int TV, Tab& tab, int start, float* buf, BackT* back, int* path, float* red,
+__device__ int viterbi_gx(const float* xs, int TV, Tab& tab, int start_, float* buf, BackT* back, int* path, float* red,
                           Hook hook = Hook(), BufHook buf_free = BufHook())
 {
     using V = VX<L, K, NT>;
@@ -350,6 +352,7 @@ __device__ int viterbi_gx(const float* xs, int TV, Tab& tab, int start, float* b
     constexpr int W = G / GW;
     constexpr int WPS = V::step_words(8 * (int)sizeof(BackT));
     const int tid = threadIdx.x;
+    const int start = __builtin_amdgcn_readfirstlane(start_);
     // every thread owns groups when there are at least NT of them (the kernels launch exactly NT threads): a
     // compile-time true then, and the step loop carries no exec-mask branches
     const bool act = V::ACT >= NT || tid < V::ACT;
@@ -404,7 +407,18 @@ __device__ int viterbi_gx(const float* xs, int TV, Tab& tab, int start, float* b
         return r;
     }();
     const int wv = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const int st0 = __builtin_amdgcn_readfirstlane(start);
+    // The savings of a fixed start hold while the unreachable states are exactly those of cost +inf. A target of 2^60 or
+    // more (or none, a NaN, as +inf) among the positions that reach only some states may take a reachable state there as
+    // well, which then ties with unreachable ones: such a search runs over all states, as one with a free start does.
+    // (Below that a cost stays finite: at most 15 such positions, squares under 2^122 for tables within 2^60.)
+    constexpr int PART = (L - 1) / K;  // positions with K (t+1) < L
+    bool partial = start >= 0;
+    if (partial) {
+        const int tl = (tid & 63) < PART ? (tid & 63) : PART - 1;
+        const uint32_t ab = (uint32_t)__float_as_int(target(tl < TV ? tl : TV - 1)) & 0x7FFFFFFFu;
+        partial = __builtin_amdgcn_ballot_w64(ab >= 0x5D800000u) == 0;  // 2^60
+    }
+    const int st0 = partial ? start : -1;
     // whether some member state of this wave is reachable at position p (always, once every state is)
     const auto wave_live = [&](int p) {
         if (!SKIP || st0 < 0 || K * (p + 1) >= L) return true;
@@ -747,10 +761,7 @@ __device__ int viterbi_gx(const float* xs, int TV, Tab& tab, int start, float* b
             for (int wv = 1; wv < NT / 64; ++wv) m = fmin(m, redp[wv]);
             s = (int)low_of(m);
         }
-        // a final cost of NaN (a NaN target: each cost of that position and
-        // every later one is NaN; in one pass the result may then come from a thread that owns no states); the
-        // reference's argmin then returns the first entry, state 0, and the traceback below stays inside the
-        // back-pointers
+        // (a state, whatever the table holds: the traceback below stays inside the back-pointers)
         s = (uint32_t)s < (uint32_t)V::NS ? s : 0;
         s = __builtin_amdgcn_readfirstlane(s);
         const auto emit = [&](int c, int sc) {

@@ -148,7 +148,7 @@ __global__ __launch_bounds__(LAMQ_WIDE_NT) void viterbi_wide_kernel(const float*
     // position 0: every state (a free first state), or the 2^k successors of the given start
     const int st0 = start ? start[row] : -1;
     {
-        const float x0 = xr[0];
+        const float x0 = search_target(xr[0]);
         for (int s = tid; s < NS; s += LAMQ_WIDE_NT) {
             const float d = x0 - C[s];
             const float q = d * d;
@@ -182,7 +182,7 @@ __global__ __launch_bounds__(LAMQ_WIDE_NT) void viterbi_wide_kernel(const float*
                 back[(int64_t)t * R + g] = (uint8_t)bh;
             }
             __syncthreads();  // every read of cost and pv done, best complete
-            const float xt = xr[t];
+            const float xt = search_target(xr[t]);
             for (int s = tid; s < NS; s += LAMQ_WIDE_NT) {
                 const float d = xt - C[s];
                 const float q = d * d;
@@ -220,7 +220,7 @@ __global__ __launch_bounds__(LAMQ_WIDE_NT) void viterbi_wide_kernel(const float*
             __syncthreads();
             // every state's new cost reads a minimum (cost[s >> k], s >> k < R) before any is overwritten (a barrier
             // between)
-            const float xt = xr[t];
+            const float xt = search_target(xr[t]);
             float nc[MAXI];
             const int spt = NS / LAMQ_WIDE_NT;
 #pragma unroll

@@ -71,9 +71,10 @@ __device__ __forceinline__ float xmc(float x, const uint32_t (&Ch)[SPT / 2], int
     return (i & 1) ? xmc_hi(x, Ch[i >> 1]) : xmc_lo(x, Ch[i >> 1]);
 }
 
-// Search one path of TV steps; thread 0 writes path[0..TV). xs: TV float32 targets. start < 0: free first state.
+// Search one path of TV steps; thread 0 writes path[0..TV). xs: TV float32 targets, through search_target
+// already or, with RAWX, as they come. start < 0: free first state.
 // xbuf: QS floats of LDS (indexed through swz). back: (TV-1)*1024 words (LDS or global). red: 32 words of LDS.
-template <int L, int K>
+template <int L, int K, bool RAWX>
 __device__ void viterbi_big(const float* xs, int TV, uint32_t (&Ch)[VBig<L, K>::SPT / 2], int start, float* xbuf,
                             uint32_t* back, int* path, float* red)
 {
@@ -89,7 +90,8 @@ __device__ void viterbi_big(const float* xs, int TV, uint32_t (&Ch)[VBig<L, K>::
             for (int g = 0; g < V::GQ; ++g)
                 bprev[q * V::GQ + g] = (rs >= 0 && q * V::RQ + V::GQ * tid + g != rs) ? __builtin_inff() : 0.0f;
     }
-    float xprev = xs[0];
+    const auto target = [&](int t) { return RAWX ? search_target(xs[t]) : xs[t]; };
+    float xprev = target(0);
     for (int t = 1; t < TV; ++t) {
         // best[j]: minimum so far of group j = q*GQ + g; hw[j]: its winning h, packed into bits [j*K, j*K+K) once per
         // step. With 16 predecessors (K = 4) hw holds h itself, an inline constant of the selects (the compiler
@@ -161,7 +163,7 @@ __device__ void viterbi_big(const float* xs, int TV, uint32_t (&Ch)[VBig<L, K>::
 #pragma unroll
         for (int j = 0; j < V::G; ++j) bprev[j] = best[j];
         back[(t - 1) * BIG_NT + tid] = bits;
-        xprev = xs[t];
+        xprev = target(t);
     }
     // final argmin, lowest state on ties (a thread's states increase with (q, i))
     float bv = __builtin_inff();
@@ -235,7 +237,7 @@ __global__ __launch_bounds__(BIG_NT) void viterbi_rows_big_kernel(const float* _
     uint32_t Ch[V::SPT / 2];
     load_half_table<L, K>(table16, Ch);
     uint32_t* back = BACK_GLOBAL ? back_ws + row * (int64_t)(T - 1) * BIG_NT : back_lds;
-    viterbi_big<L, K>(x + row * ldx, T, Ch, start ? start[row] : -1, xbuf, back, states + row * lds, red);
+    viterbi_big<L, K, true>(x + row * ldx, T, Ch, start ? start[row] : -1, xbuf, back, states + row * lds, red);
 }
 
 // minima-exchange search (trellis.h), for up to BIG_GX_MAX_R groups
@@ -357,9 +359,9 @@ __global__ __launch_bounds__(BIG_NT) void ldlq_trellis_block_big_kernel(
         const int a = (int)(ahead < look ? ahead : look);
         const int TV = w + a;
         const int jo = (int)(j - b0);
-        if (tid < TV) xs[tid] = (float)(trow[jo + tid] / Sr);
+        if (tid < TV) xs[tid] = search_target((float)(trow[jo + tid] / Sr));
         __syncthreads();
-        viterbi_big<L, K>(xs, TV, Ch, st, xbuf, back, path, red);
+        viterbi_big<L, K, false>(xs, TV, Ch, st, xbuf, back, path, red);
         if (tid < w) {
             const int p = path[tid];
             states[row * lds + j + tid] = p;

@@ -137,6 +137,55 @@ def test_viterbi_nan_and_infinite_targets_match_oracle(E, L, k):
     assert np.array_equal(got, O.viterbi(x, tab, L, k, start=st))
 
 
+BAD_TARGETS = np.concatenate([np.array([0x7FC00000, 0xFFFFFFFF, 0x7F800000, 0xFF800000], dtype=np.uint32).view(np.float32),
+                              np.array([1.5e19, -3e25, 1.2e18], dtype=np.float32)])
+
+
+@pytest.mark.parametrize("L,k", [(12, 1), (12, 2), (12, 3), (12, 4), (9, 2), (6, 4), (13, 1), (15, 3), (16, 1), (16, 2),
+                                 (16, 3), (16, 4), (10, 5)])
+@pytest.mark.parametrize("T", [3, 24, 40])
+def test_viterbi_bad_first_targets_match_oracle(E, L, k, T):
+    """NaN, infinite and huge targets (whose squares overflow, at once or in the sum of a few) at the first positions, where
+    a fixed start still reaches only some states: reachable costs are then +inf too and tie with unreachable ones."""
+    from lookatmyquant_amd.tables import quantile_table
+
+    tab = quantile_table(L, 0)
+    rng = np.random.default_rng(70 * L + 10 * k + T)
+    at = [p for p in (0, 1, 2, 3, 4, 7, 11, 15) if p < T]
+    x = rng.standard_normal((len(BAD_TARGETS) * len(at), T)).astype(np.float32)
+    for i, v in enumerate(BAD_TARGETS):
+        for j, p in enumerate(at):
+            x[i * len(at) + j, p : p + (2 if abs(v) < 1e30 else 1)] = v
+    st = rng.integers(0, 1 << L, len(x))
+    for start in (st, None):
+        say(f"viterbi L={L} k={k} T={T}, bad first targets, start {start is not None}")
+        sg = None if start is None else cuda(start, torch.int32)
+        got = E.viterbi_rows(cuda(x), cuda(tab.astype(np.float32)), L, k, start=sg).cpu().numpy()
+        assert np.array_equal(got, O.viterbi(x, tab, L, k, start=start))
+
+
+@pytest.mark.parametrize("L,k", [(12, 1), (12, 2), (12, 4), (9, 2), (16, 1), (16, 2), (16, 3), (16, 4)])
+def test_ldlq_trellis_bad_targets_match_oracle(E, L, k):
+    """The fused sweep over rows that hold a NaN, an infinity or a huge value in some column: every state is the oracle's."""
+    from lookatmyquant_amd.tables import quantile_table
+
+    tab = quantile_table(L, 0)
+    rng = np.random.default_rng(9 * L + k)
+    n = 160
+    Xa = rng.standard_normal((400, n))
+    _, U, _ = O.environment(Xa.T @ Xa / 400)
+    X = rng.standard_normal((9, n))
+    S = O.row_scale(X)
+    for r, (c, v) in enumerate([(0, np.nan), (3, np.nan), (17, np.inf), (34, -np.inf), (131, np.nan), (40, 1e25), (64, -1e300),
+                                (2, 2e19)]):
+        X[r, c] = v
+    say(f"ldlq trellis L={L} k={k}, bad targets")
+    st = E.ldlq_trellis(cuda(X), cuda(S), cuda(U), cuda(tab), L, k).cpu().numpy()
+    with np.errstate(all="ignore"):
+        want = O.ldlq_trellis(X, U, S, tab, L, k)
+    assert np.array_equal(st, want)
+
+
 @pytest.mark.parametrize("L,k,B,T", [(12, 2, 3, 33), (12, 4, 2, 580), (12, 1, 2, 600), (12, 4, 2, 1024), (12, 3, 2, 1025),
                                      (8, 2, 300, 600), (12, 2, 700, 120), (5, 1, 3, 1024)])
 def test_viterbi_back_pointer_places_match_oracle(E, L, k, B, T):
