@@ -8,9 +8,17 @@
 // Workgroups of the fused block a CU holds (four waves each, one per SIMD). A row's search alternates steps that fill
 // the vector unit with stretches of latency (a barrier and an LDS round trip per step, the traceback, the refit's chain),
 // which only other rows cover: 6,144 x 2,560 at L = 12, 1 to 4 bits: 12.6 ms with four, 11.2 with five, 10.5 with six.
-// Six is what fits: 23.8 KB of LDS (the step's rows of U take the minima's place, which are free by then, instead of
-// 16 KB of their own: four fitted) and 80 registers.
+// Six fit 23.8 KB of LDS (the step's rows of U take the minima's place, which are free by then, instead of 16 KB of their
+// own: four fitted) and 80 registers, in which k <= 2 fits whole; k = 3 at L = 12 keeps 2 registers in scratch, k = 4 12,
+// the merged kernel 16, and gains all the same (k = 4 alone at 512 columns: 2,560 rows 977 us with five and none in
+// scratch, 970 with six; 6,144 2,137, 2,048; 960 474, 496). At L = 8 .. 11 and k = 4, whose searches are shorter, six
+// would keep 22, and five are ahead (L = 8: 960 rows 371 us against 442, 2,560 765 against 904, 6,144 1,753 against
+// 1,916; L = 11: 411, 490; 878, 1,023; 1,959, 2,153) except where the rows fit one round of six and not of five (1,300 rows
+// at L = 8: 668 against 487). Below L = 8 k = 4 has few distinct minima and six are ahead again (L = 5, 6,144 rows: 1,571
+// with five, 1,368 with six).
 #define LAMQ_BLK_WAVES 6
+template <int L, int K>
+constexpr int blk_waves() { return K == 4 && L >= 8 && L < 12 ? 5 : LAMQ_BLK_WAVES; }
 
 // ------------------------------------------------------------------------------------------------
 // viterbi_rows: one workgroup per row (opgraph/codes.py:151-181).
@@ -351,7 +359,7 @@ __device__ __forceinline__ void trellis_block_row(BlkSmem<L, K>& sm, int64_t row
 }
 
 template <int L, int K>
-__global__ __launch_bounds__(LAMQ_NT, LAMQ_BLK_WAVES) void ldlq_trellis_block_kernel(
+__global__ __launch_bounds__(LAMQ_NT, (blk_waves<L, K>())) void ldlq_trellis_block_kernel(
     const double* __restrict__ T, int64_t n, int64_t ldT, const double* __restrict__ U, int64_t ldU,
     const double* __restrict__ S, const double* __restrict__ table64, const float* __restrict__ table32,
     int64_t b0, int64_t b1, int width, int look, int32_t* __restrict__ state, int32_t* __restrict__ states,
@@ -394,7 +402,7 @@ extern "C" int lamq_ldlq_trellis_block(double* T, int64_t m, int64_t n, int64_t 
 
 // ------------------------------------------------------------------------------------------------ row groups at once
 // One launch for every row group of a stage at L = 12 (the reference's fitted tables): a launch per group ends in a
-// tail of partly idle CUs (four 256-thread rows per CU, so ceil(rows / 1024) rounds), which one launch over all their
+// tail of partly idle CUs (six 256-thread rows per CU, so ceil(rows / 1536) rounds), which one launch over all their
 // rows does not have. Workgroup b takes row b of the concatenated groups (in the table's order), finds its group (a
 // uniform scan of at most LAMQ_TRELLIS_MAX_GROUPS entries) and runs that width's block in that width's LDS layout
 // over one shared array (the widest layout's size: as many workgroups per CU as for each width alone).
@@ -426,7 +434,7 @@ __global__ __launch_bounds__(LAMQ_NT, LAMQ_BLK_WAVES) void ldlq_trellis_groups_k
     const double* __restrict__ S, int64_t b0, int64_t b1, int width, int look, int32_t* __restrict__ state,
     int32_t* __restrict__ states, int64_t lds, double* __restrict__ Z, int64_t ldZ, int pre, BlkGroups groups)
 {
-    static_assert(blk_groups_smem_bytes<L>() * 6 <= 160 * 1024, "six workgroups per CU");
+    static_assert(blk_groups_smem_bytes<L>() * LAMQ_BLK_WAVES <= 160 * 1024, "LAMQ_BLK_WAVES workgroups per CU");
     __shared__ __align__(16) uint8_t raw[blk_groups_smem_bytes<L>()];
     int64_t b = blockIdx.x;
     int i = 0;
