@@ -631,24 +631,30 @@ __global__ __launch_bounds__(256) void gemm_splitk_f64_kernel(double* __restrict
 #define LAMQ_SPLITK_DEEPK 1024
 #endif
 
-// Deeper products whose 128-tiles (a LOWER one's: half of them) are fewer than this go out as 64-tiles. Measured, 128-tile
-// (or, under 128 tiles, the register kernel) against 64-tile: QEP's target (a factor and three products) of 1,024 x 2,560
-// (160 tiles) 2.87 -> 2.28 ms, 2,048 x 2,560 (320) 3.29 -> 2.63, 4,096 x 2,560 (640) 3.43 -> 3.29, 2,560 x 4,096 (640)
-// 6.53 -> 6.17; the factor at n = 1,024 / 2,560 / 4,096 655 -> 622, 1,718 -> 1,600, 3,165 -> 3,098 us. From 1,024 tiles
-// on the 128-tiles fill the chip and are ahead by up to 2% (4,096 x 4,096: 7.86 against 8.00 ms).
+// Deeper products whose 128-tiles (a LOWER one's: half of them) are fewer than this go out as 64-tiles, which need four
+// times as many for a round of the CUs and so waste less of the last one. Measured, 128-tile (or, under 128 tiles, the
+// register kernel) against 64-tile: QEP's target (a factor and three products) of 1,024 x 2,560 (160 tiles) 2.87 -> 2.28
+// ms, 2,048 x 2,560 (320) 3.29 -> 2.63, 4,096 x 2,560 (640) 3.43 -> 3.29, 2,560 x 4,096 (640) 6.53 -> 6.17; the factor at
+// n = 1,024 / 2,560 / 4,096 655 -> 622, 1,718 -> 1,600, 3,165 -> 3,098 us. From 1,024 tiles on the two are within 6%
+// either way (4,096 x 4,096 targets: 7.86 against 8.00 ms).
+// Where the last round of 128-tiles, one a CU, is filled to three quarters or more after a first, there is little left to
+// win, and the 64-tiles' second read of the operands shows: at K = 2,560, B as [k][col], 440 tiles 665 (128) and 623 us
+// (64), 480 667 and 706, 512 669 and 706, 540 1,008 and 793, 640 1,014 and 880, 720 1,016 and 1,047, 800 1,316 and 1,134,
+// 960 1,322 and 1,313, 992 1,323 and 1,396, 1,023 1,323 and 1,410. Those stay on the 128-tiles; a first round does not
+// (256 tiles: 379 and 360), nor do triangular products, whose rounds are of unequal tiles (512 tiles of 4,096 columns: 761
+// and 581; 992 1,144 and 1,092).
 #ifndef LAMQ_MID_TILES128
 #define LAMQ_MID_TILES128 1024
 #endif
 
-// TRI (LAMQ_TRI_KGE, LAMQ_TRI_KLE): op(B) is triangular and the 128-tile kernel skips the stages of its zero part (the
-// other kernels read the zeros).
+// TRI (LAMQ_TRI_KGE, LAMQ_TRI_KLE): op(B) is triangular and the 128-tile and 64-tile streaming kernels skip the stages of
+// its zero part (the other kernels read the zeros).
 template <bool TRANSB, bool LOWER, bool OVERWRITE = false, int TRI = 0>
 static int gemm_sub_f64(double* C, int64_t ldc, const double* A, int64_t lda, const double* B, int64_t ldb, int64_t M,
                         int64_t N, int64_t K, const int32_t* info, hipStream_t s)
 {
     if (M <= 0 || N <= 0 || K <= 0) return LAMQ_OK;
-    // the 128 tiles once there are enough of them to fill most of the chip, for operands it can load in 16-byte
-    // chunks
+    // operands that the streaming kernels (128 and 64 tiles) can load in 16-byte chunks
     // (a [k][col] B chunk holds columns col, col + 1: N even keeps the pair inside the row)
     const bool chunks = (lda % 2) == 0 && (ldb % 2) == 0 && (K % 2) == 0 && (TRANSB || (N % 2) == 0) &&
                         ((uintptr_t)A % 16) == 0 && ((uintptr_t)B % 16) == 0;
@@ -676,14 +682,16 @@ static int gemm_sub_f64(double* C, int64_t ldc, const double* A, int64_t lda, co
     }
     if constexpr (!OVERWRITE) {
         // (a LOWER product's 128-tiles: about half)
-        if (chunks && (LOWER ? tiles128 / 2 : tiles128) < LAMQ_MID_TILES128 && cdiv(M, 64) <= 65535) {
+        constexpr int64_t CUS = 256;
+        const bool filled = !LOWER && TRI == 0 && tiles128 > CUS && (tiles128 - 1) % CUS >= CUS * 3 / 4;
+        if (chunks && !filled && (LOWER ? tiles128 / 2 : tiles128) < LAMQ_MID_TILES128 && cdiv(M, 64) <= 65535) {
             hipLaunchKernelGGL((gemm64_f64_kernel<TRANSB, LOWER, TRI>), grid, dim3(256), 0, s, C, ldc, A, lda, B, ldb, M, N,
                                K, info);
             LAMQ_LAUNCH_CHECK();
             return LAMQ_OK;
         }
     }
-    if (!OVERWRITE && chunks && tiles128 >= 128) {
+    if (!OVERWRITE && chunks) {
         dim3 grid128((unsigned)cdiv(N, G8_BM), (unsigned)cdiv(M, G8_BM));
         hipLaunchKernelGGL((gemm128_f64_kernel<TRANSB, LOWER, G8_BK, TRI>), grid128, dim3(256), 0, s, C, ldc, A, lda, B,
                            ldb, M, N, K, info);

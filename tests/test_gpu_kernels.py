@@ -371,11 +371,15 @@ def test_gemm_sub_short_k(E, M, N, K, transb):
 @pytest.mark.parametrize("M,N,K,transb,tri", [(65, 130, 1026, False, 0), (64, 64, 1040, True, 0), (1, 2, 130, True, 0),
                                               (700, 1300, 1300, True, 1), (129, 1298, 1298, False, 2),
                                               (63, 1100, 1100, False, 1), (1000, 1026, 1026, True, 2),
-                                              (3970, 4034, 144, True, 0)])
+                                              (3970, 4034, 144, True, 0), (3801, 4034, 144, True, 0),
+                                              (3801, 4034, 144, False, 0), (2817, 4034, 144, True, 0),
+                                              (2817, 4034, 144, False, 0), (5900, 2562, 2562, True, 1),
+                                              (5900, 2562, 2562, False, 2)])
 def test_gemm_sub_64_tiles(E, M, N, K, transb, tri):
     """Deep products whose 128-tiles are too few for the chip, on the 64-tile streaming kernel: ragged M, N and K, both
     layouts and both triangular forms, C a slice of a wider matrix whose other columns stay as they are, against a
-    float64 product on the GPU."""
+    float64 product on the GPU. In 128-tiles: up to 272 in the first cases, 960 (3,801 rows) and 987 (5,900); 1,024
+    (3,970) and 736 in a nearly full last round (2,817) are the other sides of the rule, on the 128-tile kernel."""
     g = torch.Generator(device="cuda").manual_seed(M + 3 * N + 7 * K + tri)
     Cw = torch.randn(M, N + 6, generator=g, device="cuda", dtype=torch.float64)
     A = torch.randn(M, K, generator=g, device="cuda", dtype=torch.float64)
