@@ -441,7 +441,7 @@ __device__ int viterbi_gx(const float* xs, int TV, Tab& tab, int start_, float* 
     bool live = wave_live(0);
     // one step of the search, position t, reading minima buffer cur (written into cur ^ 1 with two buffers)
     const auto step = [&](const int t, int& cur) {
-        const float xn = target(t + 1);
+        const float xn = xs[t + 1];  // (search_target at the step's end, so that nothing waits for the load here)
         const int base = (SKIP && st0 >= 0 && K * (t + 1) < L)
                              ? (int)(((uint32_t)st0 << (K * (t + 1))) & (uint32_t)(V::NS - 1)) : 0;
         const bool one_h = SKIP && st0 >= 0 && K * (t + 1) <= L - K;
@@ -521,7 +521,7 @@ __device__ int viterbi_gx(const float* xs, int TV, Tab& tab, int start_, float* 
         }
         lds_barrier();
         cur ^= 1;
-        x = xn;
+        x = RAWX ? search_target(xn) : xn;
         live = wave_live(t + 1);
         if (act && live) {
 #pragma unroll

@@ -90,9 +90,9 @@ __device__ void viterbi_big(const float* xs, int TV, uint32_t (&Ch)[VBig<L, K>::
             for (int g = 0; g < V::GQ; ++g)
                 bprev[q * V::GQ + g] = (rs >= 0 && q * V::RQ + V::GQ * tid + g != rs) ? __builtin_inff() : 0.0f;
     }
-    const auto target = [&](int t) { return RAWX ? search_target(xs[t]) : xs[t]; };
-    float xprev = target(0);
+    float xprev = RAWX ? search_target(xs[0]) : xs[0];
     for (int t = 1; t < TV; ++t) {
+        const float xt = xs[t];  // (search_target at the step's end, so that nothing waits for the load here)
         // best[j]: minimum so far of group j = q*GQ + g; hw[j]: its winning h, packed into bits [j*K, j*K+K) once per
         // step. With 16 predecessors (K = 4) hw holds h itself, an inline constant of the selects (the compiler
         // schedules this form better there); otherwise h already shifted into place. With more than 16 groups a
@@ -163,7 +163,7 @@ __device__ void viterbi_big(const float* xs, int TV, uint32_t (&Ch)[VBig<L, K>::
 #pragma unroll
         for (int j = 0; j < V::G; ++j) bprev[j] = best[j];
         back[(t - 1) * BIG_NT + tid] = bits;
-        xprev = target(t);
+        xprev = RAWX ? search_target(xt) : xt;
     }
     // final argmin, lowest state on ties (a thread's states increase with (q, i))
     float bv = __builtin_inff();
