@@ -307,6 +307,8 @@ def run_c5(args):
                                     "mfma", 1e12, kt.launches("qep_gemm")),
         "rht": kernel_line(kt.ms("rht"), kt.work.get("rht", 0.0), MFMA_F64_PEAK_TFLOPS, "TFLOP/s", "mfma", 1e12,
                            kt.launches("rht")),
+        "rht_fast": kernel_line(kt.ms("rht_fast"), kt.work.get("rht_fast", 0.0), HBM_PEAK_GBS, "GB/s", "hbm", 1e9,
+                                kt.launches("rht_fast")),
         "pack_codes": kernel_line(kt.ms("pack"), kt.work.get("pack", 0.0), HBM_PEAK_GBS, "GB/s", "hbm", 1e9,
                                   kt.launches("pack")),
     }
@@ -737,8 +739,10 @@ def run_c3(args):
             "ldlq_trellis_block": trellis_line(kt.ms("block"), ops_total, kt.launches("block"), full_total),
             "trailing_update_f64": kernel_line(kt.ms("trailing"), trail_total, MFMA_F64_PEAK_TFLOPS, "TFLOP/s",
                                                "mfma", 1e12, kt.launches("trailing")),
-            "rht": kernel_line(kt.ms("rht"), kt.work["rht"], MFMA_F64_PEAK_TFLOPS, "TFLOP/s", "mfma", 1e12,
-                               kt.launches("rht"))}
+            "rht": kernel_line(kt.ms("rht"), kt.work.get("rht", 0.0), MFMA_F64_PEAK_TFLOPS, "TFLOP/s", "mfma", 1e12,
+                               kt.launches("rht")),
+            "rht_fast": kernel_line(kt.ms("rht_fast"), kt.work.get("rht_fast", 0.0), HBM_PEAK_GBS, "GB/s", "hbm", 1e9,
+                                    kt.launches("rht_fast"))}
     line = {
         "metric": METRIC, "value": round(weights / (ms * 1e-3), 1), "unit": "weights/s", "n_gpus": 1,
         "steps": args.steps, "warmup": args.warmup, "ms_per_step": round(ms, 3), "higher_is_better": True,

@@ -161,6 +161,12 @@ def rht_flops(rows: int, n: int) -> float:
     return 2.0 * rows * n * (a + b)
 
 
+def rht_work(rows: int, n: int) -> tuple:
+    """The timer key and work of rht_rows over `rows` rows of width n: ("rht", the flops of the two products) for the
+    widths that go through them, ("rht_fast", 16n bytes a row) for those of the fast transforms, which HBM bounds."""
+    return ("rht_fast", 16.0 * rows * n) if fast_factor(n) else ("rht", rht_flops(rows, n))
+
+
 @lru_cache(maxsize=64)
 def _factor_sizes(n: int) -> tuple:
     A, B = hadamard_factors(n)

@@ -280,12 +280,12 @@ def stage_statistics(Xq_chunks, w_chunks=None, Xr_chunks=None):
 
 def stage_factor(H: torch.Tensor, in_seed: int, damp: float = 0.01, timer: E.KernelTimer | None = None):
     """The stage's factor as quantize_stage_row_groups makes it: (U, dead, info) of the rotated, damped H (no host
-    synchronisation: info is a device value, 0 when positive definite). timer: spans "rht" (R H R^T: two
-    passes of rht_rows, 2n(a + b) flops a row, and a transpose) and "chol" (4n^3/3 flops)."""
+    synchronisation: info is a device value, 0 when positive definite). timer: spans "rht" or "rht_fast" (R H R^T: two
+    passes of rht_rows, rht_work's count, and a transpose) and "chol" (4n^3/3 flops)."""
     dev = E._abi.device()
     Hg = torch.as_tensor(H).to(dev, torch.float64).contiguous()
     n = Hg.shape[0]
-    with E.span(timer, "rht", 2.0 * E.rht_flops(n, n)):
+    with E.span(timer, *E.rht_work(2 * n, n)):
         Hr = E.rotate_hessian(Hg, in_seed)
     with E.span(timer, "chol", 4.0 * n ** 3 / 3):
         _, U, dead, info = E.chol_inv_upper(Hr, damp=damp, raise_on_fail=False)
@@ -307,7 +307,7 @@ def quantize_stage_row_groups(targets: dict, groups: dict, H: torch.Tensor, in_s
     check=False the caller checks the factor's info itself, after the sweep is enqueued: no host synchronisation
     here, the results then to be discarded if it failed). timer: an
     engine.KernelTimer; every launch of the sweep is timed on this stream (one stream for all groups) under "block" and
-    "trailing", the row rotations under "rht" (2n(a + b) flops a row), and the factor as in stage_factor."""
+    "trailing", the row rotations as rht_work counts them, and the factor as in stage_factor."""
     names = list(targets)
     stage_tables = {}  # the table of each width, resolved before any device work
     for bits in sorted({int(g["bits"]) for nm in names for g in groups[nm]}):
@@ -343,7 +343,7 @@ def quantize_stage_row_groups(targets: dict, groups: dict, H: torch.Tensor, in_s
     X_all, S_all = {}, {}
     for nm in names:
         W = torch.as_tensor(targets[nm]).to(dev, torch.float64).contiguous()
-        with E.span(timer, "rht", E.rht_flops(W.shape[0], W.shape[1])):
+        with E.span(timer, *E.rht_work(*W.shape)):
             X_all[nm], S_all[nm] = E.rht_rows(W, in_seed, want_rms=True)
     # rows of one width across the stage's matrices go through one sweep
     by_bits: dict = {}

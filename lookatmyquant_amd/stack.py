@@ -195,7 +195,7 @@ class StackBuild:
     raises LinAlgError, as the reference's Environment does (frame.py:521-522). kernels: an engine.KernelTimer; every
     kernel of the stages then runs on the caller's stream, one after the other, each span timed with events and
     credited with its algorithmic work ("hessian" N n (n + 1) flops, "cross_gram" 2 N n^2, "chol" 4 n^3 / 3, "rht"
-    HBM bytes, "qep_gemm", "block" trellis ops, "trailing" flops, "pack" bytes); without it the stage factor runs on a
+    flops or "rht_fast" HBM bytes (engine.rht_work), "qep_gemm", "block" trellis ops, "trailing" flops, "pack" bytes); without it the stage factor runs on a
     second stream next to the QEP targets and each stage's row groups are swept on streams of their own."""
 
     def __init__(self, tokens: torch.Tensor, sh: Shape = Shape(), token_w: torch.Tensor | None = None,
@@ -392,7 +392,7 @@ class StackBuild:
             st, Srow = res[nm]
             m, n = st.shape
             Q = _decode(st, Srow, plans[nm], self.device_tables())
-            with E.span(kt, "rht", E.rht_flops(m, n)):
+            with E.span(kt, *E.rht_work(m, n)):
                 Wh = E.rht_rows(Q, in_seed, inverse=True)
             wq[nm] = Wh.to(torch.bfloat16)
             for gp, rows in zip(plans[nm], E.device_rows(plans[nm], dev)):

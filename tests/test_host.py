@@ -308,6 +308,16 @@ def test_reachable_search_ops_match_brute_force(L, k, T, start):
         assert E.viterbi_search_ops(L, k, T) - E.viterbi_search_ops(L, k, T - 1) == E.viterbi_ops_per_row_step(L, k)
 
 
+def test_rht_work_is_of_the_kernels_that_run():
+    """The fast transforms' widths in HBM bytes (no products run there), the others in the products' flops."""
+    from lookatmyquant_amd import engine as E
+
+    for n in (1024, 1536, 2560, 4096, 8192):
+        assert E.rht_work(10, n) == ("rht_fast", 160.0 * n)
+    for n, ab in ((256, 32), (960, 76), (9728, 216)):
+        assert E.rht_work(10, n) == ("rht", 20.0 * n * ab)
+
+
 def test_trellis_block_ops_cover_every_call():
     from lookatmyquant_amd import engine as E
 
