@@ -106,7 +106,7 @@ int lamq_ldlq_multirate_block(double* T, int64_t m, int64_t n, int64_t ldT, cons
  * lamq_viterbi_rows and lamq_ldlq_trellis_block (the same references, the same arithmetic and tie rules)
  * for tables whose values are exactly representable in fp16, passed as their fp16 bit patterns
  * (table16, 4-byte aligned; table64 holds the same values in float64 for the settled values).
- * One 1024-thread workgroup per row. The fused block needs width <= 16, width + look <= 24 and
+ * One workgroup per row. The fused block needs width <= 16, width + look <= 24 and
  * b1 - b0 <= 128; the
  * standalone search keeps back-pointers of paths longer than 24 steps in the workspace:
  * lamq_viterbi16_workspace_size(B, T, L, k) bytes.

@@ -208,6 +208,7 @@ __device__ __forceinline__ double pair_min(const float (&c)[N], const LowWords<N
 // k = 4 7.27 -> 6.25).
 template <class V>
 struct TabF16Wide {
+    static_assert(V::G % 2 == 0, "members in pairs");
     float v[V::SPT];
     const uint16_t* src;
     __device__ __forceinline__ void load(const uint16_t* __restrict__ C16, int t)

@@ -492,7 +492,7 @@ __global__ __launch_bounds__(gx_nt<L>(), gx_nt<L>() / 256) void ldlq_trellis_blo
 
 // ------------------------------------------------------------------------------------------------ row groups at once
 // One launch for every row group of a stage: the groups differ in bits per weight (k), and a launch per group ends in
-// a tail of idle CUs (one 1024-thread row per CU, so ceil(rows / 256) rounds), which one launch over all their rows
+// a tail of idle CUs (one row per CU, of gx_nt threads, so ceil(rows / 256) rounds), which one launch over all their rows
 // does not have. Workgroup b takes row b of the concatenated groups, finds its group (a uniform scan of at most
 // LAMQ_TRELLIS_MAX_GROUPS entries) and runs that width's search in that width's LDS layout over one shared array.
 struct GxGroup {
