@@ -623,7 +623,10 @@ __global__ __launch_bounds__(256) void gemm_splitk_f64_kernel(double* __restrict
 // Deeper [k][col] products (K <= LAMQ_SPLITK_DEEPK) take it too where the 128-tile kernel's workgroups would fill the
 // chip's 512 slots (two a CU) poorly: fewer than LAMQ_SPLITK_TILES128 tiles, or a second round holding under 64 of
 // them. Measured at K = 512 (the sweep's deep products): 20-80 tiles 5.7-17 -> 19-35 TFLOP/s, 300-320 tiles 35-38 ->
-// 44-46, 560 tiles 43 -> 47; at 384-480 and 608 tiles the two kernels are even or the 128-tile one is ahead.
+// 44-46, 560 tiles 43 -> 47; at 384-480 and 608 tiles the two kernels are even or the 128-tile one is ahead. (The line
+// is the 128-tile kernel's. Against the 64-tile kernel below, which would take these products otherwise, at K = 512: 20
+// tiles 17 us and 27, 80 36 and 45, 128 52 and 48, 200 78 and 79, 300 111 and 98, 380 138 and 115, 560 198 and 167: the
+// order of its sums is another.)
 #ifndef LAMQ_SPLITK_TILES128
 #define LAMQ_SPLITK_TILES128 384
 #endif
